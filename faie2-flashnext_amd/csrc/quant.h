@@ -73,6 +73,18 @@ bool gemv_planes_fit(const QLayout &L);
 int gemv_launch(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, float *work,
                 size_t work_bytes, hipStream_t st, int ks_force = 0);
 
+// The GEMV on the matrix cores (quant_mx.cuh), by group of formats; rows of whole units of 256 values.  gemv_mx_use:
+// whether a weight takes it (by its format and columns alone, so that the path never depends on nt, unless
+// fn_gemv_override forces a plan of the vector kernels).
+bool gemv_mx_use(const QLayout &L);
+int gemv_mx1(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, hipStream_t st);
+int gemv_mx2(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, hipStream_t st);
+int gemv_mx3(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, hipStream_t st);
+int gemv_mx4(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, hipStream_t st);
+// the format set `kind` of quant_grp.hip, its parts in the set's order
+int gemv_mx_grp(int kind, const QLayout *const *L, const uint8_t *const *packed, float *const *y, const float *x, int nt,
+                hipStream_t st);
+
 // the GEMV with ks splits along the row and no reduce pass: part[k][t][r] = sum over split k's groups, k < *ks_out
 // (ks capped so that every split holds a group); the consumer sums the partials in split order.  The split is fixed
 // by the call, never by nt, so token t keeps the bits of a one-token call

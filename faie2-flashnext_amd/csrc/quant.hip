@@ -10,7 +10,8 @@
 //   * decoding: one lane decodes one group of 32 values into exact small-integer floats q[32] plus, per half of
 //     16 values, a scale s and an offset m, such that the GGUF value is fl(s * q - m) rounded once -- the value
 //     ggml's dequantize_row_* computes (s * q is exact for every format whose m is not zero);
-//   * GEMV: 16 lanes per row, four rows per wave, four waves per workgroup; each lane walks the row's groups
+//   * GEMV: on the matrix cores for most shapes (quant_mx.cuh; gemv_mx_use), else, or when a plan is forced, on the
+//     vector units: 16 lanes per row, four rows per wave, four waves per workgroup; each lane walks the row's groups
 //     with stride 16, keeps the next group's loads in flight while it does the current one's FMAs, and the row
 //     sum is a 16-lane DPP reduction.  Short rows split K over workgroups whose partials a second pass adds in a
 //     fixed order, so results do not depend on timing.  For formats without an offset the scale multiplies the
@@ -172,6 +173,19 @@ bool gemv_planes_fit(const QLayout &L) {
     return true;
 }
 
+// Rows of 4 to 32 whole units of 256 values: below, a workgroup would be fewer than 4 waves for a tile; above, the waves
+// (at most 16) would hold more than two units of x, for which the registers do not reach.  A BF16 unit takes 128 bytes
+// of a lane, so two of them do not fit beside x either.  The other formats (the routed experts') have no decode there.
+bool gemv_mx_use(const QLayout &L) {
+    if (g_ov_lpr || g_ov_kernel || L.cols % 256 || L.cols < 4 * 256 || L.cols > 32 * 256) return false;
+    switch (L.type) {
+        case QT_BF16: return L.cols <= 16 * 256;
+        case QT_Q8_0: case QT_IQ4_NL: case QT_IQ4_XS: case QT_Q4_K: case QT_Q5_K: case QT_Q6_K:
+        case QT_IQ3_S: return true;
+        default: return false;
+    }
+}
+
 int gemv_launch(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, float *work,
                 size_t work_bytes, hipStream_t st, int ks_force) {
     if (nt < 1 || nt > MAXNT) FN_FAIL("gemv: nt must be 1..8");
@@ -179,6 +193,14 @@ int gemv_launch(const QLayout &L, const uint8_t *packed, const float *x, int nt,
     if (!gemv_planes_fit(L)) FN_FAIL("gemv: a plane of the packed weight exceeds 4 GiB");
     if ((uintptr_t) packed % 16 || (uintptr_t) x % 16) FN_FAIL("gemv: weight and x must be 16-byte aligned");
     const GemvPlan pl = gemv_plan(L, ks_force);
+    if (pl.ks == 1 && gemv_mx_use(L)) {
+        switch (L.type) {
+            case QT_BF16: case QT_Q8_0: return gemv_mx1(L, packed, x, nt, y, st);
+            case QT_IQ4_NL: case QT_IQ4_XS: return gemv_mx2(L, packed, x, nt, y, st);
+            case QT_Q4_K: case QT_Q5_K: return gemv_mx3(L, packed, x, nt, y, st);
+            default: return gemv_mx4(L, packed, x, nt, y, st);
+        }
+    }
     float *out = y;
     if (pl.ks > 1) {
         const size_t need = (size_t) pl.ks * nt * L.rows * 4;

@@ -67,6 +67,20 @@ int gemv_group_launch(const GemvPart *parts, int n, const float *x, int nt, hipS
             if (gemv_launch(*parts[i].L, parts[i].packed, x, nt, parts[i].y, nullptr, 0, st, 1)) return -1;
         return 0;
     }
+    // on the matrix cores (one unit of x a wave, so up to 4096 columns): every part with its own GEMV's bits.  All the
+    // sets' formats take that path or none does: it goes by the columns.
+    if (gemv_mx_use(*parts[0].L) && parts[0].L->cols <= 16 * 256) {
+        const QLayout *L[4];
+        const uint8_t *pk[4];
+        float *y[4];
+        if ((uintptr_t) x % 16) FN_FAIL("gemv: weight and x must be 16-byte aligned");
+        for (int s = 0; s < n; ++s) {
+            const GemvPart &g = parts[slot_of[s]];
+            if ((uintptr_t) g.packed % 16) FN_FAIL("gemv: weight and x must be 16-byte aligned");
+            L[s] = g.L, pk[s] = g.packed, y[s] = g.y;
+        }
+        return gemv_mx_grp(kind, L, pk, y, x, nt, st);
+    }
     // lanes per row: the fewest any part's own plan takes, at least 32 (the group is built for 32 and 64)
     int lpr = 64;
     const QLayout *L[4];

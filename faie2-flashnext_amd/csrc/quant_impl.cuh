@@ -1101,6 +1101,7 @@ struct GPart {
     PP P;
     int rows, nwg;
     float *out;
+    int rt;  // (quant_mx.cuh) rows of a tile
 };
 template <int N> struct GParts {
     GPart p[N];
@@ -1159,7 +1160,7 @@ int gemv_grp_nt(const QLayout *const *L, const PP *P, float *const *y, const flo
     for (int i = 0; i < N; ++i) {
         int w = need[i];
         if (sum_need > budget) w = std::min(need[i], std::max(1, (int) (budget * (double) L[i]->bytes / bytes)));
-        ps.p[i] = GPart{P[i], L[i]->rows, w, y[i]};
+        ps.p[i] = GPart{P[i], L[i]->rows, w, y[i], 0};
         nwg += w;
     }
     hipLaunchKernelGGL((k_gemv_grp<NT, LPR, TS...>), dim3((unsigned) nwg), dim3(512), lds, st, ps, G, x, L[0]->cols);

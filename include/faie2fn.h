@@ -52,8 +52,10 @@ int fn_test_dequant(uint32_t type, const uint8_t *W, int rows, int cols, float *
  * ks: split-K workgroups per row, as the reference's (out[2]).  tb: not the reference's tiles per block (the
  * workgroups here are fixed at 8 waves) but this library's kernel choice (1 x staged in chunks, 2 x staged once,
  * 3 / 4 x staged once with the deep / short walk).  warps_per_sm: the resident waves per CU a persistent grid is
- * sized for (the reference's target warps per SM).  Lanes per row and ks > 1 change the summation order, the other
- * choices give the same bits.  The model forward's GEMVs take no split-K whatever ks asks (no work buffer). */
+ * sized for (the reference's target warps per SM).  A forced wpt, ks > 1 or tb takes the vector kernels; without one,
+ * most shapes run on the matrix cores, which sum in an order of their own (the same to about 1e-7).  Lanes per row and
+ * ks > 1 change the summation order, the other choices give the same bits among themselves.  The model forward's GEMVs
+ * take no split-K whatever ks asks (no work buffer). */
 void fn_gemv_override(int wpt, int ks, int tb, int warps_per_sm);             /* faie2fn.cu:2786 */
 /* The reference's persistent-grid switch: waves != 0 (default) launches the GEMV on the workgroups resident at once,
  * each walking many row tiles; 0 launches one workgroup per row tile.  Same bits either way; fn_gemv_plan's out[5]
@@ -74,7 +76,8 @@ void fn_moe_override(int gu_wpt, int gu_tb, int dn_wpt, int dn_tb);           /*
  * out = {values per group (32), 16-lane groups per row (wpt, as fn_gemv_override takes it), split-K workgroups per
  * row, rows per workgroup pass, waves per workgroup (8), workgroups along the rows (0 = persistent grid: the
  * workgroups resident at once, sized at launch; after fn_gemv_waves(0) one per row tile of rows-per-pass rows),
- * groups per row}.  Like the reference's it depends on the shape only, never on the number of tokens. */
+ * groups per row}, of the vector kernels (which a forced plan takes).  Like the reference's it depends on the shape
+ * only, never on the number of tokens. */
 int fn_gemv_plan(uint32_t type, int rows, int cols, int *out);                /* faie2fn.cu:2809 */
 void fn_bench_hot(int on);                                                    /* faie2fn.cu:2822 */
 /* ms per GEMV call of nt tokens (1..8) on random bytes of the format, iters calls replayed as one hipGraph, each
@@ -344,9 +347,10 @@ int fn_gemv_dev(uint32_t type, const uint8_t *packed, int rows, int cols, const 
  * activation row as separate GEMVs, faie2fn.cu:2386-2403): y[i] [nt][rows[i]] = W_i x for i < n (1..4).  One
  * launch, x staged once per workgroup, when the formats form one of the built sets ({IQ4_XS, IQ3_S, BF16},
  * {IQ4_XS, Q6_K, BF16}, {IQ4_XS, IQ4_XS, Q6_K, BF16}, in any order) and x of nt tokens fits the LDS; otherwise one
- * fn_gemv_dev-like launch per weight.  A grouped launch sums each row over at least 32 lanes, so a weight whose own
- * plan takes 16 lanes per row may differ from fn_gemv_dev in the last bits; the path taken depends on the formats
- * and shapes only, never on nt (token t gets the bits of a one-token call).  No work buffer. */
+ * fn_gemv_dev-like launch per weight.  On the matrix cores (cols 1024 to 4096) a weight gets fn_gemv_dev's bits; the
+ * vector kernels' grouped launch sums each row over at least 32 lanes, so a weight whose own plan takes 16 lanes per row
+ * may differ there in the last bits.  The path taken depends on the formats and shapes only, never on nt (token t gets
+ * the bits of a one-token call).  No work buffer. */
 int fn_gemv_group_dev(int n, const uint32_t *types, const int *rows, int cols, const uint8_t *const *packed,
                       const float *x, int nt, float *const *y, void *stream);
 

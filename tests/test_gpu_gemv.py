@@ -323,3 +323,73 @@ def test_gemv_group_path_independent_of_nt(fnlib):
             assert np.array_equal(y[i], y1[0]), (t, i)
             assert np.array_equal(y1, fnlib.gemv(t, raw, r, cols, x[i:i + 1])), (t, i)
 
+
+
+# The matrix-core GEMV (csrc/quant_mx.cuh): rows at the edges of its tiles (4, 8 and 16 rows), columns at the edges of
+# its wave splits (units of 256 values: 4, 12 / 13, 16 / 17 with an odd last unit, 24 / 25, 32) and one unit outside them
+# (3 and 33, the vector kernels), calls at the edges of its token tiles (4 / 5).
+MX_TYPES = ["BF16", "Q8_0", "IQ4_NL", "IQ4_XS", "Q4_K", "Q5_K", "Q6_K", "IQ3_S"]
+MX_SHAPES = [(1, 1024), (17, 3072), (511, 3328), (513, 1024), (1025, 4096), (5, 4352), (33, 6144), (16, 6400), (35, 8192),
+             (2049, 1280), (9, 768), (9, 8448)]
+
+
+@pytest.mark.parametrize("name", MX_TYPES)
+@pytest.mark.parametrize("rows,cols", MX_SHAPES)
+def test_gemv_matrix_cores(fnlib, name, rows, cols):
+    """Against float64 and against the vector kernels (a forced plan), on an x with outliers; tokens independent of the
+    call they are in.  Bound: products are exact and sums are 32-bit, at most 264 groups deep, so 264 / 2 roundings of
+    2^-24 against the largest partial sum (1e-5 holds for every path; 2e-6 is four times what either path shows)."""
+    t = TYPES[name]
+    rng = np.random.default_rng(rows * 7 + cols)
+    _say(f"gemv matrix cores {name} {rows}x{cols}")
+    raw = random_finite(t, rows, cols, rng)
+    if t != TYPES["BF16"]:
+        blk = raw.reshape(-1, oracle.qblock(t)[1])   # scales of one size: a row's error is its own
+        for b in {8: [1], 20: [1], 21: [1], 23: [1], 12: [1, 3], 13: [1, 3], 14: [209]}[t]:
+            blk[:, b] = 0x20
+    else:
+        raw = (rng.standard_normal(rows * cols).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).view(np.uint8)
+    x = rng.standard_normal((8, cols)).astype(np.float32)
+    x[5] *= np.exp(2 * rng.standard_normal(cols)).astype(np.float32)
+    x[6] *= np.float32(1e-30)
+    ref = oracle.gemv(t, raw, rows, cols, x)
+    y = fnlib.gemv(t, raw, rows, cols, x)
+    fnlib.gemv_override(kernel=4)
+    try:
+        yv = fnlib.gemv(t, raw, rows, cols, x)
+    finally:
+        fnlib.gemv_override(0)
+    for i in range(8):
+        scale = np.abs(ref[i]).max() if rows > 8 else np.abs(x[i].astype(np.float64)).max() * np.abs(
+            oracle.dequant(t, raw, rows, cols)).max() * np.sqrt(cols)
+        assert np.abs(y[i] - ref[i]).max() <= 2e-6 * scale, i
+        assert np.abs(y[i] - yv[i]).max() <= 4e-6 * scale, i
+    for nt in (1, 3, 4, 5):
+        assert np.array_equal(fnlib.gemv(t, raw, rows, cols, x[:nt]), y[:nt]), nt
+
+
+@pytest.mark.parametrize("name", ["BF16", "Q8_0", "IQ4_XS", "IQ3_S", "Q5_K"])
+def test_gemv_matrix_cores_specials(fnlib, name):
+    """Infinities and NaNs in x (and in a BF16 weight) come out where the vector kernels put them; a token beside them is
+    untouched."""
+    t, rows, cols = TYPES[name], 40, 2560
+    rng = np.random.default_rng(11)
+    _say(f"gemv matrix cores, infinities and NaNs, {name} {rows}x{cols}")
+    raw = random_finite(t, rows, cols, rng)
+    if t == TYPES["BF16"]:
+        w = (rng.standard_normal(rows * cols).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        w[3 * cols + 7], w[5 * cols + 9], w[6 * cols + 11] = 0x7F80, 0xFF80, 0x7FC0  # inf, -inf, NaN
+        raw = w.view(np.uint8)
+    x = rng.standard_normal((4, cols)).astype(np.float32)
+    clean = fnlib.gemv(t, raw, rows, cols, x)
+    x[1, 100], x[2, 200], x[3, 300] = np.inf, -np.inf, np.nan
+    y = fnlib.gemv(t, raw, rows, cols, x)
+    fnlib.gemv_override(kernel=4)
+    try:
+        yv = fnlib.gemv(t, raw, rows, cols, x)
+    finally:
+        fnlib.gemv_override(0)
+    assert np.array_equal(y[0].view(np.uint32), clean[0].view(np.uint32))
+    assert np.array_equal(np.isnan(y), np.isnan(yv))
+    inf = np.isinf(yv)
+    assert np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], yv[inf])
