@@ -20,7 +20,7 @@
 //   * The combine kernel merges the splits with the log-sum-exp identity and applies o / L * sigmoid(gate).
 // Device cache layouts (max_ctx a multiple of 64):
 //   Kc: [B][nkv][max_ctx / 64][hd / 4][64][4]   Vc: [B][nkv][max_ctx][hd]
-#include "qsa.h"
+#include "attn_prep.cuh"
 
 #include <algorithm>
 #include <cmath>
@@ -29,70 +29,12 @@ namespace fn {
 
 namespace {
 
-constexpr int HD = 256;     // head dim built (the reference's, faie2fn.cu:49)
-constexpr int TILE = 64;    // keys per tile (= wave size)
 constexpr int WAVES = 4;
-constexpr int MAXROT = 128;
 
-
-struct AttnArgs {
-    int B, nq, nkv, nt, max_ctx, nsplit, nrot;
-    float eps;
-    const int32_t *pos;
-    const float *qg, *knew, *vnew, *wq, *wk;
-    float *Kc, *Vc;
-    float *Q;        // [B nt][nkv][HD/4][grp][4]
-    float *part_o;   // [B nt][nq][nsplit][HD]
-    float *part_ml;  // [B nt][nq][nsplit][2]
-    float *og;
-    const int32_t *keys;   // visible-key list per query (QSA) or null (dense)
-    const int32_t *nkeys;
-    int kstride;           // list stride per query
-    unsigned *status;      // per-device status word: FN_STATUS_POS when a new token falls outside the cache
-    float inv_freq[MAXROT / 2];
-};
-
-__device__ __forceinline__ size_t k_index(int max_ctx, int b, int nkv, int g, int p, int d) {
-    const size_t tile = ((size_t) b * nkv + g) * (max_ctx / TILE) + p / TILE;
-    return ((tile * (HD / 4) + d / 4) * TILE + (p % TILE)) * 4 + (d % 4);
-}
-
-// RMSNorm + RoPE of the query heads and the new key (faie2fn.cu:1451-1478), cache append.
 // grid (B nt, nq + nkv), HD threads
 __global__ void __launch_bounds__(HD) k_attn_prep(const AttnArgs a) {
-    __shared__ float buf[HD];
-    __shared__ float red[HD / 64];
-    const int bt = blockIdx.x, b = bt / a.nt, t = bt - b * a.nt, j = blockIdx.y, d = threadIdx.x;
-    const int P = a.pos[b] + t;
-    if (P < 0 || P >= a.max_ctx) {  // outside the cache: nothing is written past it; the status word says so
-        if (j == 0 && d == 0) atomicOr(a.status, FN_STATUS_POS);
-        return;
-    }
-    const bool isq = j < a.nq;
-    const int g = isq ? j / (a.nq / a.nkv) : j - a.nq;
-    const float x = isq ? a.qg[((size_t) bt * a.nq + j) * 2 * HD + d] : a.knew[((size_t) bt * a.nkv + g) * HD + d];
-    const float ws = wave_sum(x * x);
-    if ((d & 63) == 0) red[d >> 6] = ws;
-    __syncthreads();
-    const float ss = red[0] + red[1] + red[2] + red[3];
-    buf[d] = x * rsqrtf(ss / HD + a.eps) * (isq ? a.wq[d] : a.wk[d]);
-    __syncthreads();
-    float y = buf[d];
-    const int half = a.nrot / 2;
-    if (d < a.nrot) {
-        const int i = d < half ? d : d - half;
-        const float x0 = buf[i], x1 = buf[i + half];
-        const float ang = (float) P * a.inv_freq[i];  // fp32 angle (faie2fn.cu:1440)
-        const float cs = cosf(ang), sn = sinf(ang);
-        y = d < half ? x0 * cs - x1 * sn : x1 * cs + x0 * sn;
-    }
-    if (isq) {
-        const int grp = a.nq / a.nkv, hh = j - g * grp;
-        a.Q[((((size_t) bt * a.nkv + g) * (HD / 4) + d / 4) * grp + hh) * 4 + (d % 4)] = y;
-    } else {
-        a.Kc[k_index(a.max_ctx, b, a.nkv, g, P, d)] = y;
-        a.Vc[(((size_t) b * a.nkv + g) * a.max_ctx + P) * HD + d] = a.vnew[((size_t) bt * a.nkv + g) * HD + d];
-    }
+    __shared__ float buf[HD + HD / 64];
+    attn_prep_row(a, blockIdx.x, blockIdx.y, buf);
 }
 
 // Split-K attention partials.  grid (nsplit, nkv, B nt), WAVES*64 threads.
@@ -961,14 +903,11 @@ int attn_qsa_launch(const AttnDecode &p, const QsaIndexer &ix, hipStream_t st) {
         FN_FAIL("attn_qsa: workspace too small");
     const int grp = p.nq / p.nkv;
     if (grp != 4 && grp != 8 && grp != 12) FN_FAIL("attn: query heads per kv head must be 4, 8 or 12");
-    const int32_t *keys = nullptr, *nkeys = nullptr;
-    float *iwork = reinterpret_cast<float *>(reinterpret_cast<char *>(p.work) + (aw + 255) / 256 * 256);
-    if (qsa_select_launch(ix, iwork, p.work_bytes - (aw + 255) / 256 * 256, &keys, &nkeys, st)) return -1;
     AttnArgs a{};
     a.B = p.B; a.nq = p.nq; a.nkv = p.nkv; a.nt = p.nt; a.max_ctx = p.max_ctx; a.nsplit = p.nsplit;
     a.nrot = p.nrot; a.eps = p.eps; a.pos = p.pos; a.qg = p.qg; a.knew = p.k; a.vnew = p.v; a.wq = p.wq;
     a.wk = p.wk; a.Kc = p.Kc; a.Vc = p.Vc; a.og = p.og;
-    a.keys = keys; a.nkeys = nkeys; a.kstride = ix.top * 4 + 4;
+    a.kstride = ix.top * 4 + 4;
     if (p.status) a.status = p.status;
     else if (status_word(&a.status)) return -1;
     const size_t bt = (size_t) p.B * p.nt;
@@ -977,14 +916,20 @@ int attn_qsa_launch(const AttnDecode &p, const QsaIndexer &ix, hipStream_t st) {
     a.part_ml = a.part_o + bt * p.nq * p.nsplit * HD;
     for (int i = 0; i < p.nrot / 2; ++i)
         a.inv_freq[i] = (float) (1.0 / std::pow((double) p.theta, (double) (2 * i) / p.nrot));
+    const int32_t *keys = nullptr, *nkeys = nullptr;
+    float *iwork = reinterpret_cast<float *>(reinterpret_cast<char *>(p.work) + (aw + 255) / 256 * 256);
+    if (qsa_select_launch(ix, iwork, p.work_bytes - (aw + 255) / 256 * 256, &keys, &nkeys, &a, st)) return -1;
+    a.keys = keys; a.nkeys = nkeys;
     const dim3 sg(p.nsplit, p.nkv, (unsigned) bt), sb(WAVES * 64);
     if (p.nt == 1) {  // q norm + RoPE and the K/V append folded into the split kernel
         if (grp == 8) hipLaunchKernelGGL((k_attn_split<8, true, true>), sg, sb, 0, st, a);
         else if (grp == 12) hipLaunchKernelGGL((k_attn_split<12, true, true>), sg, sb, 0, st, a);
         else hipLaunchKernelGGL((k_attn_split<4, true, true>), sg, sb, 0, st, a);
     } else {
-        hipLaunchKernelGGL(k_attn_prep, dim3((unsigned) bt, p.nq + p.nkv), dim3(HD), 0, st, a);
-        stage_mark(st);
+        if (!qsa_prep_folds(p.nt)) {
+            hipLaunchKernelGGL(k_attn_prep, dim3((unsigned) bt, p.nq + p.nkv), dim3(HD), 0, st, a);
+            stage_mark(st);
+        }
         if (grp == 8) hipLaunchKernelGGL((k_attn_split<8, false, true>), sg, sb, 0, st, a);
         else if (grp == 12) hipLaunchKernelGGL((k_attn_split<12, false, true>), sg, sb, 0, st, a);
         else hipLaunchKernelGGL((k_attn_split<4, false, true>), sg, sb, 0, st, a);

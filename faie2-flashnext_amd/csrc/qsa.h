@@ -17,9 +17,13 @@ struct QsaIndexer {
 };
 
 size_t qsa_work_bytes(int B, int nt, int max_ctx, int top);
-// indexer prep + scores + selection; on return *keys / *nkeys point into work (visible-key list per query)
+// Calls of 2 to this many tokens have the prep of the indexer and of the attention inside the scoring launch
+inline bool qsa_prep_folds(int nt) { return nt > 1 && nt <= 16; }
+// indexer prep + scores + selection; on return *keys / *nkeys point into work (visible-key list per query).  Where
+// qsa_prep_folds, the scoring launch also does the attention's prep (the query rows and the K/V append) from at.
+struct AttnArgs;
 int qsa_select_launch(const QsaIndexer &p, float *work, size_t work_bytes, const int32_t **keys, const int32_t **nkeys,
-                      hipStream_t st);
+                      const AttnArgs *at, hipStream_t st);
 int qsa_blocks_launch(const QsaIndexer &p, int j0, int j1, hipStream_t st);
 
 // sparse GQA decode: the attention of AttnDecode restricted to the keys the indexer selects

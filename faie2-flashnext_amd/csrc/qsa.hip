@@ -4,25 +4,25 @@
 //                call completes get their block key rope(rmsnorm(mean of 4 raw keys) * wkn) at the block start
 //   k_ix_blocks  the same block keys over a range of blocks (prefill / rebuilding a cache)
 //   k_ix_score   score(block j) = sum over the 4 heads of relu(q_h . BK_j) / sqrt(128); lane = block over a
-//                block-tiled key store, so each wave load is one coalesced 1 KiB row of 64 blocks.  For one-token
-//                calls k_ix_prep's work runs inside it (k_ix_score<true>), one dependent launch fewer
+//                block-tiled key store, so each wave load is one coalesced 1 KiB row of 64 blocks.  For calls of up
+//                to 16 tokens k_ix_prep's work runs inside it, and from 2 tokens the attention's prep too
 //   k_ix_select  the top `top` blocks by score, ties at the threshold kept lowest index first, by a 3-pass radix
 //                select on the score bits in LDS histograms (the reference binary-searches 32 bit-passes); it emits
 //                the sorted list of visible keys (kept blocks, then the incomplete tail) that the attention split
 //                kernel gathers from.  A query with <= top complete blocks gets the dense list 0..pos.
 // Device layouts: IKc [B][max_ctx][128]; BKc [B][max_ctx/4/64][32][64][4] (64 blocks x 128 dims per tile; max_ctx a
 // multiple of 256).
-#include "qsa.h"
+#include "attn_prep.cuh"
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace fn {
 
 namespace {
 
 constexpr int IXH = 4, IXD = 128, IXR = 4, BT = 64;  // heads, head dim, keys per block, blocks per tile
-constexpr int MAXROT = 128;
 
 struct IxArgs {
     int B, nt, max_ctx, top, nrot;
@@ -35,6 +35,7 @@ struct IxArgs {
     int32_t *keys;   // [B nt][top * IXR + IXR]
     int32_t *nkeys;  // [B nt]
     int j0, j1;      // block range of k_ix_blocks
+    int G;           // scoring workgroups a query
     unsigned *status;  // per-device status word (FN_STATUS_POS)
     float inv_freq[MAXROT / 2];
 };
@@ -125,40 +126,62 @@ __global__ void __launch_bounds__(256) k_ix_blocks(const IxArgs a) {
     if (j < a.j1) block_key(a, b, j, buf[wave], lane);
 }
 
-// grid (B nt, G), 256 threads.  Workgroup y takes tiles y, y + G, ... of 64 blocks; lane = block, and wave w loads
-// dims 32w .. 32w+31 of the tile (8 coalesced 1 KiB rows), so one tile is 4 waves' loads in flight at once.  The
+// grid (B nt, G [+ nq + nkv]), 256 threads.  Workgroup y < G takes tiles y, y + G, ... of 64 blocks; lane = block, and
+// wave w loads dims 32w .. 32w+31 of the tile (8 coalesced 1 KiB rows), so one tile is 4 waves' loads in flight at once.  The
 // four waves' partial head dots meet in LDS; wave 0 applies the relu per head and stores the tile's 64 scores.
-// PREP (one-token calls, nt = 1): k_ix_prep's work rides in this launch.  Every workgroup of a query normalises and
-// ropes the 4 index q heads itself (wave h = head h, as k_ix_prep), with its first tile's loads already in flight;
-// workgroup 0 appends the raw index key; when the new key completes block jn, the workgroup owning jn's tile
-// (y = (jn / 64) % G) builds the block key from the 3 cached raw keys and the new one (the same arithmetic as
-// block_key), stores it, and scores block jn from its own copy: no workgroup reads a block key this launch writes.
-// Both happen before the dense test, so a dense query's caches are kept up to date.  Same bits as k_ix_prep followed
-// by the plain kernel.
-template <bool PREP>
-__global__ void __launch_bounds__(256) k_ix_score(const IxArgs a) {
+// PREP (1 to 16 tokens): k_ix_prep's work rides in this launch.  Every workgroup of a query
+// normalises and ropes the 4 index q heads itself (wave h = head h, as k_ix_prep), with its first tile's loads already
+// in flight; workgroup 0 appends the raw index key.  The blocks that the call's keys up to this query's own complete
+// are built by the workgroups owning their tiles (y = (j / 64) % G), one a wave, from cached raw keys and, for the
+// call's own, the rows of iqk (the same bits and the same arithmetic as block_key): no workgroup reads a raw or block
+// key that this launch writes.  Each scores those blocks from its own copy; the query whose key completes the block
+// stores it.  All of it before the dense test, so a dense query's caches are kept up to date.  Same bits as k_ix_prep
+// followed by the plain kernel.
+// ATTN (2 to 16 tokens, at most 4 new blocks): more workgroups a query, one for each query head and each key / value
+// head of the attention, do its prep (attn_prep_row): nothing here depends on it, and two dependent launches go, one
+// of them a serial walk over the tokens on one workgroup a sequence.  Measured on MI355X, the layer step at 4
+// sequences of 16K, 4 tokens, 24 / 2 heads: 90.0 -> 83.0 us (the three launches 10.4 + 10.1 + 4.8 us, this one 14.7);
+// 1 sequence of 4K, 8 tokens: 16.2 + 5.4 + 4.6 -> 7.3 us.  Past 16 tokens more than four blocks could be new, and the
+// launches of their own remain.
+constexpr int MAXNEW = 4;
+struct NoAttn {};
+template <bool PREP, class AT = NoAttn>
+__global__ void __launch_bounds__(256) k_ix_score(const IxArgs a, const AT at) {
+    constexpr bool ATTN = std::is_same<AT, AttnArgs>::value;
     constexpr int CW = IXD / 4 / 4;  // float4 chunks per wave
     __shared__ float4 qs[IXD / 4][IXH];
     __shared__ float part[2][4][IXH][BT];
-    __shared__ float buf[PREP ? 4 : 1][IXD];  // PREP: the waves' RoPE rows; row 0 then holds the new block key
+    __shared__ float buf[PREP ? MAXNEW : 1][IXD];  // PREP: the waves' RoPE rows, then the new block keys
     const int bt = blockIdx.x, b = bt / a.nt, t = bt - b * a.nt;
+    if constexpr (ATTN) {
+        if ((int) blockIdx.y >= a.G) {
+            attn_prep_row(at, bt, blockIdx.y - a.G, &part[0][0][0][0]);
+            return;
+        }
+    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int P = a.pos[b] + t;
+    const int pos = a.pos[b], P = pos + t;
     const int nb = min(P + 1, a.max_ctx) / IXR;
     const int ntiles = (nb + BT - 1) / BT;
     int tile = blockIdx.y;
     const bool live = nb > a.top && tile < ntiles;  // sparse query, and this workgroup has tiles
-    // PREP: the head's query row, the new raw key and the 3 cached raw keys of the block the new key would complete
-    // requested first (unconditional, clamped), so that the query's norm and RoPE wait for them and not for the tile
-    float2 x, nk, rk[IXR - 1];
+    const int jnew = max(pos, 0) / IXR, jw = jnew + (ATTN ? wave : 0);
+    // PREP: blocks jnew .. nb - 1 are new (one token: at most one, wave 0's), block jw is this wave's
+    // PREP: the head's query row, the new raw key and the raw keys of the wave's new block requested first
+    // (unconditional, clamped), so that the query's norm and RoPE wait for them and not for the tile
+    float2 x, nk, rk[IXR];
     if constexpr (PREP) {
         const float *row = a.iqk + (size_t) bt * (IXH * IXD + IXD);
         x = reinterpret_cast<const float2 *>(row + wave * IXD)[lane];
         nk = reinterpret_cast<const float2 *>(row + IXH * IXD)[lane];
-        const int pc = min(max(P, 0), a.max_ctx - 1);
-        const float *k = a.IKc + ((size_t) b * a.max_ctx + (size_t) (pc / IXR) * IXR) * IXD;
 #pragma unroll
-        for (int e = 0; e < IXR - 1; ++e) rk[e] = reinterpret_cast<const float2 *>(k + e * IXD)[lane];
+        for (int e = 0; e < (ATTN ? IXR : IXR - 1); ++e) {
+            const int k = min(jw, a.max_ctx / IXR - 1) * IXR + e, kt = min(k - max(pos, -MAXNEW * IXR), t);
+            const float *p = !ATTN || k < pos ? a.IKc + ((size_t) b * a.max_ctx + k) * IXD
+                                              : a.iqk + ((size_t) b * a.nt + kt) * (IXH * IXD + IXD) + IXH * IXD;
+            rk[e] = reinterpret_cast<const float2 *>(p)[lane];
+        }
+        if (!ATTN) rk[IXR - 1] = nk;  // (a one-token call's key can only be its block's last)
     }
     __builtin_amdgcn_sched_barrier(0);
     const float4 *Bb = reinterpret_cast<const float4 *>(a.BKc) +
@@ -168,36 +191,34 @@ __global__ void __launch_bounds__(256) k_ix_score(const IxArgs a) {
 #pragma unroll
         for (int c = 0; c < CW; ++c) kf[c] = ld_nt(&Bb[((size_t) tile * (IXD / 4) + c) * BT]);
     }
-    int jn = -1;  // PREP: the block this call's key completes, when this workgroup builds it
     if constexpr (PREP) {
         const bool valid = P >= 0 && P < a.max_ctx;
         if (!valid) {  // past the cache: nothing to append; the status word says so
             if (blockIdx.y == 0 && threadIdx.x == 0) atomicOr(a.status, FN_STATUS_POS);
-        } else {
-            if (blockIdx.y == 0 && wave == 0)
-                reinterpret_cast<float2 *>(a.IKc + ((size_t) b * a.max_ctx + P) * IXD)[lane] = nk;
-            if ((P + 1) % IXR == 0 && (P / IXR / BT) % (int) gridDim.y == (int) blockIdx.y) jn = P / IXR;
+        } else if (blockIdx.y == 0 && wave == 0) {
+            reinterpret_cast<float2 *>(a.IKc + ((size_t) b * a.max_ctx + P) * IXD)[lane] = nk;
         }
         const float2 y = norm_rope_row(x, a.wqn, buf[wave], lane, P, a.nrot, a.inv_freq, a.eps);
         float *qf = reinterpret_cast<float *>(qs);
         qf[((2 * lane / 4) * IXH + wave) * 4 + (2 * lane) % 4] = y.x;
         qf[((2 * lane / 4) * IXH + wave) * 4 + (2 * lane) % 4 + 1] = y.y;
-        if (jn >= 0 && wave == 0) {  // (uniform in the wave)
-            // block_key's sum: the 4 raw keys in order, the last one the new key (its cached copy's bits)
+        if (jw < nb && (jw / BT) % a.G == (int) blockIdx.y && (ATTN || wave == 0)) {  // (uniform in the wave)
+            // block_key's sum: the 4 raw keys in order
             float2 sm = make_float2(0.0f, 0.0f);
 #pragma unroll
             for (int e = 0; e < IXR; ++e) {
-                const float2 v = e < IXR - 1 ? rk[e] : nk;
-                sm.x += v.x;
-                sm.y += v.y;
+                sm.x += rk[e].x;
+                sm.y += rk[e].y;
             }
             sm.x /= IXR;
             sm.y /= IXR;
-            const float2 bk = norm_rope_row(sm, a.wkn, buf[0], lane, jn * IXR, a.nrot, a.inv_freq, a.eps);
-            a.BKc[bk_index(a.max_ctx, b, jn, 2 * lane)] = bk.x;
-            a.BKc[bk_index(a.max_ctx, b, jn, 2 * lane + 1)] = bk.y;
-            buf[0][2 * lane] = bk.x;
-            buf[0][2 * lane + 1] = bk.y;
+            const float2 bk = norm_rope_row(sm, a.wkn, buf[wave], lane, jw * IXR, a.nrot, a.inv_freq, a.eps);
+            if (valid && P == jw * IXR + IXR - 1) {
+                a.BKc[bk_index(a.max_ctx, b, jw, 2 * lane)] = bk.x;
+                a.BKc[bk_index(a.max_ctx, b, jw, 2 * lane + 1)] = bk.y;
+            }
+            buf[wave][2 * lane] = bk.x;
+            buf[wave][2 * lane + 1] = bk.y;
         }
     }
     if (!live) return;  // (after the appends: a dense query's caches still grow)
@@ -210,11 +231,14 @@ __global__ void __launch_bounds__(256) k_ix_score(const IxArgs a) {
     __syncthreads();
     const float inv = 1.0f / sqrtf((float) IXD);
     float *out = a.scores + (size_t) bt * (a.max_ctx / IXR);
-    for (int it = 0; tile < ntiles; tile += gridDim.y, ++it) {
-        if (PREP && jn >= 0 && tile == jn / BT && lane == jn % BT) {  // block jn from this workgroup's own copy
+    for (int it = 0; tile < ntiles; tile += a.G, ++it) {
+        if (PREP && jnew < nb && tile >= jnew / BT) {  // (uniform) the new blocks from this workgroup's own copies
+            const int jl = tile * BT + lane;
+            if (jl >= jnew && jl < nb) {
 #pragma unroll
-            for (int c = 0; c < CW; ++c)
-                kf[c] = reinterpret_cast<const float4 *>(buf[0])[wave * CW + c];
+                for (int c = 0; c < CW; ++c)
+                    kf[c] = reinterpret_cast<const float4 *>(buf[jl - jnew])[wave * CW + c];
+            }
         }
         float s[IXH] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -227,7 +251,7 @@ __global__ void __launch_bounds__(256) k_ix_score(const IxArgs a) {
                 s[h] = fmaf(q.z, kf[c].z, s[h]);
                 s[h] = fmaf(q.w, kf[c].w, s[h]);
             }
-        const int next = tile + gridDim.y;
+        const int next = tile + a.G;
         if (next < ntiles) {
 #pragma unroll
             for (int c = 0; c < CW; ++c) kf[c] = ld_nt(&Bb[((size_t) next * (IXD / 4) + c) * BT]);
@@ -508,7 +532,7 @@ size_t qsa_work_bytes(int B, int nt, int max_ctx, int top) {
 }
 
 int qsa_select_launch(const QsaIndexer &p, float *work, size_t work_bytes, const int32_t **keys, const int32_t **nkeys,
-                      hipStream_t st) {
+                      const AttnArgs *at, hipStream_t st) {
     if (check(p)) return -1;
     if (!p.pos || !p.iqk || !p.wqn || !p.wkn || !p.IKc || !p.BKc || !work) FN_FAIL("qsa: null pointer");
     if (work_bytes < qsa_work_bytes(p.B, p.nt, p.max_ctx, p.top)) FN_FAIL("qsa: workspace too small");
@@ -524,14 +548,18 @@ int qsa_select_launch(const QsaIndexer &p, float *work, size_t work_bytes, const
     *nkeys = a.nkeys;
     // about 1024 workgroups of scoring over all queries, at most one per tile
     const int tiles = p.max_ctx / IXR / BT;
-    const int G = (int) std::max<size_t>(1, std::min<size_t>(tiles, (1024 + bt - 1) / bt));
+    a.G = (int) std::max<size_t>(1, std::min<size_t>(tiles, (1024 + bt - 1) / bt));
     const int nbmax = p.max_ctx / IXR;
+    const dim3 g((unsigned) bt, a.G);
     if (p.nt == 1) {  // the prep inside the scoring launch
-        hipLaunchKernelGGL(k_ix_score<true>, dim3((unsigned) bt, G), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(k_ix_score<true>, g, dim3(256), 0, st, a, NoAttn{});
+    } else if (qsa_prep_folds(p.nt)) {  // and the attention's
+        hipLaunchKernelGGL((k_ix_score<true, AttnArgs>), dim3((unsigned) bt, a.G + at->nq + at->nkv), dim3(256), 0, st,
+                           a, *at);
     } else {
         hipLaunchKernelGGL(k_ix_prep, dim3(p.B), dim3(256), 0, st, a);
         stage_mark(st);
-        hipLaunchKernelGGL(k_ix_score<false>, dim3((unsigned) bt, G), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(k_ix_score<false>, g, dim3(256), 0, st, a, NoAttn{});
     }
     stage_mark(st);
     if (nbmax <= 1024 * 8)

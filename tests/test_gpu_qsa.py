@@ -283,3 +283,63 @@ def test_qsa_position_outside_cache_sets_status(fnlib):
         assert np.array_equal(ik[0, :p0], ik0[0, :p0])
         for x in (K, V, IK, BK, work, og, *d.values()):
             x.free()
+
+
+@pytest.mark.parametrize("pos", [(253, 699, 126), (244, 127, 750), (511, 2, 766)])
+def test_qsa_prep_folded_same_bits(fnlib, pos):
+    """Calls of up to 16 tokens run the indexer's and the attention's prep inside the scoring launch; 17 tokens run
+    them as their own launches.  A query sees only the keys up to its own, so the first nt tokens of the 17 must give
+    the same bits: outputs, appended keys and values, raw keys and block keys.  Positions complete blocks on both
+    sides of a block tile's edge (256), stay dense (2, 126), turn sparse inside the call (top 32: 132) and run past
+    the cache's end (750, 766 of 768; those queries have no defined output)."""
+    B, nq, nkv, hd, max_ctx, top = 3, 16, 2, 256, 768, 32
+    fnlib.dev_status()  # (clears bits earlier tests left)
+    rng = np.random.default_rng(21)
+    x = {n: rng.standard_normal((B, 17) + s).astype(np.float32)
+         for n, s in (("qg", (nq, 2, hd)), ("k", (nkv, hd)), ("v", (nkv, hd)), ("iqk", (640,)))}
+    w = {n: hiprt.Buf.like(rng.normal(1.0, 0.1, m).astype(np.float32))
+         for n, m in (("wq", hd), ("wk", hd), ("wqn", 128), ("wkn", 128))}
+    cache, ikn = B * nkv * max_ctx * hd, B * max_ctx * 128
+    nsplit = 2
+
+    def call(nt):
+        _say(f"qsa prep folded: nt={nt} pos={pos}")
+        d = {"K": hiprt.Buf.empty((cache,)), "V": hiprt.Buf.empty((cache,)), "IK": hiprt.Buf.empty((ikn,)),
+             "BK": hiprt.Buf.empty((ikn // 4,)), "og": hiprt.Buf.empty((B, nt, nq, hd)),
+             "pos": hiprt.Buf.like(np.array(pos, np.int32))}
+        for j, key in enumerate(("K", "V", "IK")):
+            fnlib.fill_normal_dev(d[key].ptr, d[key].nbytes // 4, 70 + j)
+        d["BK"].zero()
+        for b, p in enumerate(pos):  # the block keys complete before the call; those of its own stay unbuilt
+            fnlib.ix_blocks_dev(1, max_ctx, 0, p // 4, d["IK"].ptr + b * max_ctx * 512, w["wkn"].ptr,
+                                d["BK"].ptr + b * max_ctx * 128)
+        y = {n: hiprt.Buf.like(np.ascontiguousarray(v[:, :nt])) for n, v in x.items()}
+        wb = fnlib.attn_qsa_work_bytes(B, nq, nt, nsplit, max_ctx, top)
+        work = hiprt.Buf(wb)
+        work.zero()
+        fnlib.attn_qsa_dev(B, nq, nkv, nt, max_ctx, d["pos"].ptr, y["qg"].ptr, y["k"].ptr, y["v"].ptr, w["wq"].ptr,
+                           w["wk"].ptr, d["K"].ptr, d["V"].ptr, y["iqk"].ptr, w["wqn"].ptr, w["wkn"].ptr,
+                           d["IK"].ptr, d["BK"].ptr, top, nsplit, work.ptr, wb, d["og"].ptr)
+        hiprt.sync()
+        out = {"og": d["og"].download(), "K": d["K"].download((B, nkv, max_ctx // 64, 64, 64, 4)),
+               "V": d["V"].download((B, nkv, max_ctx, hd)), "IK": d["IK"].download((B, max_ctx, 128)),
+               "BK": d["BK"].download((B, max_ctx // 256, 32, 64, 4))}
+        out["K"] = out["K"].transpose(0, 1, 2, 4, 3, 5).reshape(B, nkv, max_ctx, hd)
+        out["BK"] = out["BK"].transpose(0, 1, 3, 2, 4).reshape(B, max_ctx // 4, 128)
+        for b in (work, *d.values(), *y.values()):
+            b.free()
+        return out
+
+    want = call(17)
+    for nt in (2, 3, 4, 5, 8, 16):
+        got = call(nt)
+        for b, p in enumerate(pos):
+            n = min(nt, max_ctx - p)
+            assert np.array_equal(got["og"][b, :n], want["og"][b, :n]), (nt, b)
+            assert np.array_equal(got["K"][b, :, :p + n], want["K"][b, :, :p + n]), (nt, b)
+            assert np.array_equal(got["V"][b, :, :p + n], want["V"][b, :, :p + n]), (nt, b)
+            assert np.array_equal(got["IK"][b, :p + n], want["IK"][b, :p + n]), (nt, b)
+            assert np.array_equal(got["BK"][b, :(p + n) // 4], want["BK"][b, :(p + n) // 4]), (nt, b)
+    assert (fnlib.dev_status() != 0) == (max(pos) + 17 > max_ctx)
+    for b in w.values():
+        b.free()
