@@ -286,8 +286,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_attn_split(const AttnArgs a) {
 //
 // For nt > 1 the nt * GRP query rows of a (sequence, kv head) form a small matrix (R = nt * GRP rows), so the work is
 // two thin GEMMs per key block instead of R dot products, and every token reads the same K/V.  k_attn_split_mt reads
-// each K/V byte of its split once for all R rows and runs the products on v_mfma_f32_16x16x4f32, in fp32 like the
-// single-token kernel.  Both products are taken transposed so that one lane holds one query row throughout:
+// each K/V byte of its split once for all R rows and runs the products on the matrix cores, at fp32 precision like the
+// single-token kernel: here on v_mfma_f32_16x16x4f32, from 17 rows on in bf16 parts (attn_mx.cuh).  Both products are taken transposed so that one lane holds one query row throughout:
 //   S^T[key][row] = sum_d K[key][d] Q[row][d]      A = K (lane: key l%16, dim slot l/16), B = Q (lane: row l%16)
 //   O^T[d][row]  += sum_key V[key][d] P[row][key]  A = V (lane: dim l%16, key slot l/16), B = P (lane: row l%16)
 // The S^T result leaves lane l with row l%16 and keys 4(l/16)..4(l/16)+3 of the 16-key block, which is exactly the
@@ -306,10 +306,11 @@ __global__ void __launch_bounds__(WAVES * 64) k_attn_split(const AttnArgs a) {
 // One row block per wave (R <= 16): two 16-key blocks of K and V in flight while the other is multiplied.  Two row
 // blocks: twice the products per block, so half a block in flight suffices, and the walk is software pipelined --
 // the softmax step of block i is cut into stages woven between the score products of block i + 1.
-// Measured on MI355X (B = 16, 32K context, 16 query / 2 kv heads): with the K/V loads made cache-resident the layer
-// step is only 5-6 % faster, so the kernel is bound by the matrix cores and the instructions between them, not by
-// HBM: at nt = 8 the products alone take 490 us at the 2.14 GHz this load runs at, the kernel ~700 us.  Two waves per
-// SIMD with one row block each were slower (each wave loads K/V for its own 16 rows: twice the loads).
+// Measured on MI355X (B = 16, 32K context, 16 query / 2 kv heads): with the K/V loads made cache-resident the fp32 layer
+// step is only 5-6 % faster, so the fp32 walk is bound by the matrix cores and the instructions between them, not by
+// HBM: at nt = 8 its products alone take 490 us at the 2.14 GHz this load runs at, the layer step 667 us (521 in bf16
+// parts).  Two waves per SIMD with one row block each were slower (each wave loads K/V for its own 16 rows: twice the
+// loads).
 constexpr int MT_OS = HD + 4;  // LDS row stride (floats) of the merge buffer: a wave's 16 rows land on distinct banks
 constexpr float MT_SLACK = 8.0f;  // growth of a row's max (natural-log units) that triggers a rescale
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -551,54 +552,11 @@ __device__ __forceinline__ void mt_block(const float4 (&k)[16], const float4 (&v
     mt_pv<NRW>(v, p, o);
 }
 
-// grid (nsplit, nkv, B), RW * KW <= 4 waves; dynamic LDS: max(RW * NRW * 16 KiB of Q, RW * KW * 16 * MT_OS * 4 B);
-// KEEP = RW > 1 (row groups share each block through the L2)
+// the fp32 walk of one wave: its nw 16-key blocks (kw, kw + KW, ...) of the split's keys from k0
 template <int NRW, bool KEEP>
-__global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
-k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
-    extern __shared__ float4 mt_lds[];
-    __shared__ float2 mls[WAVES][NRW * 16];
-    const int sp_i = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nth = RW * KW * 64, rw = wave / KW, kw = wave - rw * KW;
-    const int R = a.nt * grp;
-    const int P0 = a.pos[b];
-    const int nkmax = min(P0 + a.nt, a.max_ctx);  // keys visible to the last token
-    const int ntiles = nkmax > 0 ? (nkmax + TILE - 1) / TILE : 0;
-    const int per = (ntiles + a.nsplit - 1) / a.nsplit;
-    const int tile0 = min(sp_i * per, ntiles), tile1 = min(tile0 + per, ntiles);
-    const int k0 = tile0 * TILE, k1 = min(tile1 * TILE, nkmax);
-    const int nblk = k1 > k0 ? (k1 - k0 + 15) / 16 : 0;
-    const int nw = nblk > kw ? (nblk - 1 - kw) / KW + 1 : 0;  // this wave's blocks
-
-    // Q of all row blocks into LDS: [row block][u][lane] float4, lane l = (row l%16, chunk 4u + l/16); rows >= R zero
-    const float4 *Qg = reinterpret_cast<const float4 *>(a.Q);
-    for (int i = tid; i < RW * NRW * 1024; i += nth) {
-        const int rb = i >> 10, u = (i >> 6) & 15, l = i & 63;
-        const int row = rb * 16 + (l & 15), c = 4 * u + (l >> 4);
-        float4 qv = f4(0.0f);
-        if (row < R) {
-            const int t = row / grp, h = row - t * grp;
-            qv = Qg[(((size_t) (b * a.nt + t) * a.nkv + g) * (HD / 4) + c) * grp + h];
-        }
-        mt_lds[i] = qv;
-    }
-    __syncthreads();
-    const float4 *qs = mt_lds + rw * NRW * 1024;
-    const float4 *Kb = reinterpret_cast<const float4 *>(a.Kc + ((size_t) b * a.nkv + g) * a.max_ctx * HD);
-    const float4 *Vb = reinterpret_cast<const float4 *>(a.Vc + ((size_t) b * a.nkv + g) * a.max_ctx * HD);
-    v4f o[NRW][16];
-    float m[NRW], l[NRW];
-    int lim[NRW];
-#pragma unroll
-    for (int j = 0; j < NRW; ++j) {
-        m[j] = -INFINITY;
-        l[j] = 0.0f;
-        const int t = min(((rw * NRW + j) * 16 + (lane & 15)) / grp, a.nt - 1);
-        lim[j] = min(min(P0 + t + 1, a.max_ctx), k1);
-#pragma unroll
-        for (int t2 = 0; t2 < 16; ++t2) o[j][t2] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+__device__ __forceinline__ void mt_walk(const float4 *Kb, const float4 *Vb, const float4 *qs, int k0, int kw, int KW,
+                                        int nw, int nkmax, int lane, v4f (&o)[NRW][16], float (&m)[NRW],
+                                        float (&l)[NRW], const int (&lim)[NRW]) {
     if (nw > 0 && NRW == 1) {
         // one row block: two whole blocks in flight (pairs of blocks; an odd count gets one block past k1, fully
         // masked, to keep the loop free of conditionals, which keeps the wait counts exact: A's loads are awaited
@@ -659,6 +617,124 @@ k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
         mt_softmax<NRW>(S, kbl(i), m, l, lim, lane, p, corr);
         mt_rescale<NRW>(o, corr);
         mt_pv<NRW>(vf, p, o);
+    }
+}
+
+#include "attn_mx.cuh"
+
+// grid (nsplit, nkv, B), RW * KW <= 4 waves; dynamic LDS: max(RW * NRW * 16 KiB of Q, RW * KW * 16 * MT_OS * 4 B), MX:
+// 24 KiB of Q a row block; KEEP = RW > 1 (row groups share each block through the L2)
+// MX: the walk on the bf16 matrix cores (attn_mx.cuh); a split whose sums hold a NaN is walked again in fp32, so that
+// infinities and NaN in the inputs give what the fp32 walk gives.
+template <int NRW, bool KEEP, bool MX>
+__global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
+    extern __shared__ float4 mt_lds[];
+    __shared__ float2 mls[WAVES][NRW * 16];
+    const int sp_i = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nth = RW * KW * 64, rw = wave / KW, kw = wave - rw * KW;
+    const int R = a.nt * grp;
+    const int P0 = a.pos[b];
+    const int nkmax = min(P0 + a.nt, a.max_ctx);  // keys visible to the last token
+    const int ntiles = nkmax > 0 ? (nkmax + TILE - 1) / TILE : 0;
+    const int per = (ntiles + a.nsplit - 1) / a.nsplit;
+    const int tile0 = min(sp_i * per, ntiles), tile1 = min(tile0 + per, ntiles);
+    const int k0 = tile0 * TILE, k1 = min(tile1 * TILE, nkmax);
+
+    const float4 *Kb = reinterpret_cast<const float4 *>(a.Kc + ((size_t) b * a.nkv + g) * a.max_ctx * HD);
+    const float4 *Vb = reinterpret_cast<const float4 *>(a.Vc + ((size_t) b * a.nkv + g) * a.max_ctx * HD);
+    v4f o[NRW][16];
+    float m[NRW], l[NRW];
+    int lim[NRW];
+#pragma unroll
+    for (int j = 0; j < NRW; ++j) {
+        const int t = min(((rw * NRW + j) * 16 + (lane & 15)) / grp, a.nt - 1);
+        lim[j] = min(min(P0 + t + 1, a.max_ctx), k1);
+    }
+    const float4 *Qg = reinterpret_cast<const float4 *>(a.Q);
+    auto q_chunk = [&](int row, int c) {  // rows >= R are zero
+        if (row >= R) return f4(0.0f);
+        const int t = row / grp, h = row - t * grp;
+        return Qg[(((size_t) (b * a.nt + t) * a.nkv + g) * (HD / 4) + c) * grp + h];
+    };
+    auto reset = [&]() {
+#pragma unroll
+        for (int j = 0; j < NRW; ++j) {
+            m[j] = -INFINITY;
+            l[j] = 0.0f;
+#pragma unroll
+            for (int t2 = 0; t2 < 16; ++t2) o[j][t2] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    };
+    reset();
+    auto walk_f32 = [&]() {
+        // Q of all row blocks into LDS: [row block][u][lane] float4, lane l = (row l%16, chunk 4u + l/16)
+        for (int i = tid; i < RW * NRW * 1024; i += nth)
+            mt_lds[i] = q_chunk((i >> 10) * 16 + (i & 15), 4 * ((i >> 6) & 15) + ((i >> 4) & 3));
+        __syncthreads();
+        const int nblk = k1 > k0 ? (k1 - k0 + 15) / 16 : 0;
+        const int nw = nblk > kw ? (nblk - 1 - kw) / KW + 1 : 0;  // this wave's blocks
+        const float4 *qs = mt_lds + rw * NRW * 1024;
+        if constexpr (!MX) {
+            mt_walk<NRW, KEEP>(Kb, Vb, qs, k0, kw, KW, nw, nkmax, lane, o, m, l, lim);
+        } else {  // the rare second walk: one block at a time, in few registers
+            for (int i = 0; i < nw; ++i) {
+                const int kb = k0 + (kw + i * KW) * 16;
+                float4 kf[16], vf[16];
+                mt_load_k<true>(kf, Kb, kb, nkmax, lane);
+                mt_load_v<true>(vf, Vb, kb, nkmax, lane);
+                mt_block<NRW>(kf, vf, kb, qs, o, m, l, lim, lane);
+            }
+        }
+    };
+    if constexpr (MX) {
+        // Q in parts: [row block][u][part][lane] of 8 bf16, lane l = (row l%16, chunks 8u + l/16 and 8u + 4 + l/16)
+        v4u *qd = reinterpret_cast<v4u *>(mt_lds);
+        for (int i = tid; i < RW * NRW * 512; i += nth) {
+            const int rb = i >> 9, u = (i >> 6) & 7, ln = i & 63, row = rb * 16 + (ln & 15), c = 8 * u + (ln >> 4);
+            const float4 x0 = q_chunk(row, c), x1 = q_chunk(row, c + 4);
+            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            Mx3 d;
+            mx_split(x, d);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) qd[rb * MX_QB + (u * 3 + p) * 64 + ln] = d.p[p];
+        }
+        __syncthreads();
+        const int nblk = k1 > k0 ? (k1 - k0 + 31) / 32 : 0;
+        const int nw = nblk > kw ? (nblk - 1 - kw) / KW + 1 : 0;  // this wave's blocks of 32 keys
+        bool bad = false;
+        if (nw > 0) {
+            MxWalk<KEEP> w;
+            w.Kb = reinterpret_cast<const char *>(Kb), w.Vb = reinterpret_cast<const char *>(Vb);
+            w.qs = qd + rw * NRW * MX_QB;
+            w.nkmax = nkmax, w.lane = lane;
+#pragma unroll
+            for (int j = 0; j < NRW; ++j) {
+                w.m[j] = m[j], w.l[j] = l[j], w.lim[j] = lim[j];
+#pragma unroll
+                for (int t2 = 0; t2 < 16; ++t2) w.o[j][t2] = o[j][t2];
+            }
+            w.walk(k0 + kw * 32, KW * 32, nw);
+#pragma unroll
+            for (int j = 0; j < NRW; ++j) {
+                m[j] = w.m[j], l[j] = w.l[j];
+                float s = l[j];
+#pragma unroll
+                for (int t2 = 0; t2 < 16; ++t2) {
+                    o[j][t2] = w.o[j][t2];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s = fmaf(o[j][t2][r], 0.0f, s);  // an infinity becomes a NaN too
+                }
+                bad |= s != s;
+            }
+        }
+        if (__syncthreads_or(bad)) {
+            reset();
+            walk_f32();
+        }
+    } else {
+        walk_f32();
     }
 
     // merge the KW key streams of each row group (log-sum-exp), then write the split partials
@@ -867,11 +943,15 @@ int attn_decode_launch(const AttnDecode &p, hipStream_t st) {
     } else if (nr <= 8 && p.B <= 65535) {
         // rows in groups of NRW 16-row blocks (RW groups), KW key streams per group, at most 4 waves
         const int nrw = nr == 1 ? 1 : 2, rw = (nr + nrw - 1) / nrw, kw = std::max(1, WAVES / rw);
-        const size_t lds = std::max((size_t) rw * nrw * 16 * HD * 4, (size_t) rw * kw * 16 * MT_OS * 4);
+        // bf16 parts wherever they fit: Q in parts takes 48 KiB of LDS a row group of 32 (three of four), and the walk's
+        // offsets into a head's cache have 32 bits
+        const bool mx = nrw == MX_NRW && rw <= 3 && p.max_ctx <= MX_MAXCTX;
+        const size_t lds = std::max((size_t) rw * nrw * (mx ? MX_QB * 16 : 16 * HD * 4), (size_t) rw * kw * 16 * MT_OS * 4);
         const dim3 mg(p.nsplit, p.nkv, p.B), mb(rw * kw * 64);
-        if (nrw == 1) hipLaunchKernelGGL((k_attn_split_mt<1, false>), mg, mb, lds, st, a, grp, rw, kw);
-        else if (rw == 1) hipLaunchKernelGGL((k_attn_split_mt<2, false>), mg, mb, lds, st, a, grp, rw, kw);
-        else hipLaunchKernelGGL((k_attn_split_mt<2, true>), mg, mb, lds, st, a, grp, rw, kw);
+        if (nrw == 1) hipLaunchKernelGGL((k_attn_split_mt<1, false, false>), mg, mb, lds, st, a, grp, rw, kw);
+        else if (mx && rw == 1) hipLaunchKernelGGL((k_attn_split_mt<2, false, true>), mg, mb, lds, st, a, grp, rw, kw);
+        else if (mx) hipLaunchKernelGGL((k_attn_split_mt<2, true, true>), mg, mb, lds, st, a, grp, rw, kw);
+        else hipLaunchKernelGGL((k_attn_split_mt<2, true, false>), mg, mb, lds, st, a, grp, rw, kw);
     } else {
         if (grp == 8) hipLaunchKernelGGL((k_attn_split<8, false>), sg, sb, 0, st, a);
         else if (grp == 12) hipLaunchKernelGGL((k_attn_split<12, false>), sg, sb, 0, st, a);

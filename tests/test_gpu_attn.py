@@ -110,6 +110,43 @@ def test_attn_multi_token_split_invariant(fnlib):
         assert oracle.relerr(o, outs[0]) <= 2e-6
 
 
+# Keys of the one split: 1, 2 and 3 blocks of 32 a wave and waves without one, a block's first and last key, with 17 to
+# 96 query rows (one to three row groups).  A result is a softmax-weighted mean of V: 256-term fp32 dot products of
+# unit-variance rows (score error about 16 * 2^-24, x 1/16 scale) and fp32 sums leave a few 1e-7 normwise; 2e-6 is ten
+# times that.
+@pytest.mark.parametrize("nq,nt", [(16, 3), (16, 4), (24, 4), (16, 8), (24, 8)])
+@pytest.mark.parametrize("keys", [8, 31, 32, 33, 65, 127, 128, 129, 257, 384])
+def test_attn_bf16_parts_walk(fnlib, nq, nt, keys):
+    _say(f"attn bf16 parts nq={nq} nt={nt} keys={keys}")
+    case = _mt_case(2, nq, 2, nt, [keys - nt, max(0, keys // 2 - nt)], 384, seed=keys * 10 + nt)
+    og = _check(fnlib, case, nsplit=1)
+    ref, _, _ = oracle.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc, case.Vc, case.pos)
+    assert oracle.relerr(og, ref) <= 2e-6
+
+
+@pytest.mark.parametrize("nq,nt", [(16, 4), (24, 8)])
+def test_attn_multi_token_infinities(fnlib, nq, nt):
+    """A cached key with an infinite element (minus infinity as a score leaves the key out, plus infinity gives NaN)
+    and a cached value with one (its dim becomes infinite), as an fp32 walk has them."""
+    _say(f"attn multi-token infinities nq={nq} nt={nt}")
+    case = _mt_case(3, nq, 2, nt, [500, 300, 200], 512, seed=5 + nq)
+    case.Kc[0, 77, :, 200] = -np.inf
+    case.Vc[1, 100, :, 33] = np.inf
+    og = fnlib.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc.copy(), case.Vc.copy(), case.pos)
+    with np.errstate(all="ignore"):
+        clean = _mt_case(3, nq, 2, nt, [500, 300, 200], 512, seed=5 + nq)
+        ref, _, _ = oracle.attn(clean.qg, clean.k, clean.v, clean.wq, clean.wk, clean.Kc, clean.Vc, clean.pos)
+    og = np.asarray(og).reshape(3, nt, nq, 256)
+    ref = np.asarray(ref).reshape(3, nt, nq, 256)
+    q = case.qg[0, :, :, 0, 200] * case.wq[200]      # dim 200 is past the rotated ones: the sign is the normed query's
+    assert np.isnan(og[0][q < 0]).all() and np.isfinite(og[0][q > 0]).all()
+    got, want = og[0][q > 0].astype(np.float64), ref[0][q > 0]
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 0.2  # one key of 500 fewer
+    assert np.isposinf(og[1][..., 33]).all()
+    rest = np.arange(256) != 33
+    assert oracle.relerr(og[1][..., rest], ref[1][..., rest]) <= TOL and oracle.relerr(og[2], ref[2]) <= TOL
+
+
 @pytest.mark.parametrize("nq,nt", [(16, 4), (16, 2), (24, 8)])
 def test_attn_multi_token_growing_scores(fnlib, nq, nt):
     """Scores that grow along the context (key scale 1 -> 21) and one outlier key 40x: the running max of every row
