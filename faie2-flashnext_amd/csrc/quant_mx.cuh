@@ -619,7 +619,6 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
     mx_tab_fill<TY>(tab, tid, blockDim.x);
     v4u f[UPW][NTILE][8];
     int xexp[UPW][NTILE];
-    const int rounds = nt - t0 > 2 ? 2 : 1;
     const bool one = mx_one<TY>(NTILE) && nt - t0 == 1;
 #pragma unroll
     for (int k = 0; k < UPW; ++k)
@@ -627,7 +626,7 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
         for (int i = 0; i < NTILE; ++i) {
             float *s = sums + (k * NTILE + i) * SUMS;
             if (one) xr[k][i].split1(lane, mine, f[k][i]);
-            else xr[k][i].split(rounds, lane, mine, f[k][i], s, xexp[k][i]);
+            else xr[k][i].split(nt - t0 - 4 * i > 2 ? 2 : 1, lane, mine, f[k][i], s, xexp[k][i]);
         }
     if constexpr (HALF) load(blk, 0, wa, false, true);
     if constexpr (UPW == 2) load(blk, 1, wb);

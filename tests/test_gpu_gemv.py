@@ -393,3 +393,17 @@ def test_gemv_matrix_cores_specials(fnlib, name):
     assert np.array_equal(np.isnan(y), np.isnan(yv))
     inf = np.isinf(yv)
     assert np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], yv[inf])
+
+
+@pytest.mark.parametrize("name", MX_TYPES)
+def test_gemv_matrix_cores_short_second_tile(fnlib, name):
+    """Calls whose second token tile is short (5, 6 and 7 tokens): every token has the bits of the 8-token call, so
+    nothing that such a tile does not load reaches a result."""
+    t, rows, cols = TYPES[name], 65, 2560
+    _say(f"gemv matrix cores, 5 to 7 tokens, {name} {rows}x{cols}")
+    rng = np.random.default_rng(12)
+    raw = random_finite(t, rows, cols, rng)
+    x = rng.standard_normal((8, cols)).astype(np.float32)
+    y = fnlib.gemv(t, raw, rows, cols, x)
+    for nt in (5, 6, 7):
+        assert np.array_equal(fnlib.gemv(t, raw, rows, cols, x[:nt]).view(np.uint32), y[:nt].view(np.uint32)), nt
