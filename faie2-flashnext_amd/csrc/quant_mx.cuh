@@ -7,7 +7,8 @@
 //   * weights: every format's codes are small integers (or the bf16 values themselves), exact in bf16.  The group's
 //     scale multiplies the 32-value dot product afterwards, in fp32, as on the VALU.
 //   * x: an fp32 value is the exact sum of three bf16 values (hi = its first 8 significant bits, mid the next 8, lo
-//     the last 8), so that every product is exact and the sums are fp32: nothing of x is rounded away.
+//     the last 8), so that every product is exact and the sums are fp32: nothing of x is rounded away.  (Values too
+//     small for bf16 to hold all three are scaled by a power of two first, MxX::split.)
 //   * tile: x is the A operand, 16 rows = 4 tokens x {hi, mid, lo, unused}; 16 weight rows are the B operand.  Lane
 //     (r, c) = (lane % 16, lane / 16) of the result holds hi, mid and lo of token c for weight row r, so that the
 //     scale, the sum of the three and the accumulator are one lane's: no shuffle anywhere.
@@ -36,6 +37,8 @@
 #pragma once
 
 #include "quant_impl.cuh"
+
+#include <type_traits>
 
 namespace fn {
 namespace {
@@ -369,20 +372,22 @@ template <uint32_t TY> constexpr int mx_lds(int W, int upw, int ntile) {
     return mx_tab_bytes<TY>() + W * mx_wave<TY>(upw, ntile) + 2 * 16 * ntile * 256;
 }
 
-// x = hi + mid + lo, exactly, each in the high 16 bits of a float (lo's low bits are zero by construction).  An
+// x = hi + mid + lo, each in the high 16 bits of a float: exact from |x| = 2^-110 on, where lo's low bits are zero by
+// construction.  Below, bf16 ends (its smallest value is 2^-133) and lo's low bits are what it does not hold.  An
 // infinity or NaN is all in hi.
 __device__ __forceinline__ void split3(float x, uint32_t &h, uint32_t &m, uint32_t &l) {
-    x = __builtin_canonicalizef(x);  // (a quiet NaN stays one without its low bits)
+    x = __builtin_canonicalizef(x);  // (a quiet NaN stays one without its low bits; folded into the product x comes from)
     h = __float_as_uint(x) & 0xFFFF0000u;
     float r = x - __uint_as_float(h);
-    r = __builtin_isfinite(x) ? r : 0.0f;
+    r = __builtin_amdgcn_fmed3f(r, r, 0.0f);  // (r; 0 where r is a NaN, of an infinity or a NaN)
     m = __float_as_uint(r) & 0xFFFF0000u;
     l = __float_as_uint(r - __uint_as_float(m));
 }
 
-__device__ __forceinline__ void split8(const float *v, v4u &h, v4u &m, v4u &l) {
+// N values (4 or 8) in pairs
+template <int N> __device__ __forceinline__ void split_n(const float *v, uint32_t *h, uint32_t *m, uint32_t *l) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < N / 2; ++k) {
         uint32_t h0, m0, l0, h1, m1, l1;
         split3(v[2 * k], h0, m0, l0);
         split3(v[2 * k + 1], h1, m1, l1);
@@ -398,10 +403,17 @@ template <uint32_t TY> constexpr bool mx_one(int ntile) { return ntile == 1 && !
 // it, split() makes the wave's A operands of it.  f[j] is lane (m, q)'s operand of group j: row m = token m / 4, part
 // m % 4 (the unused fourth row reads lo again).  Two tokens a round through the wave's LDS, 8 values a lane.
 //   sums (MIN), in the LDS: [token][group] of x (SUB: [token][group][half]);
-//   xexp (DEN): x is scaled by 2^xexp before the split.
+//   xexp: the scale of x, a power of two, by unit and token.  DEN: x is scaled by 2^xexp, of the unit's largest.  Else
+//   xexp is the mask of the result's lanes (16 a token) whose unit is scaled by 2^UP, because all of it is below 2^-63, so
+//   that values too small for an exact split (split3) have one.  A unit with a larger value is not scaled: what it may
+//   lose is below 2^-133, 2^-70 of that value.  No sum overflows by it: scaled values are below 2^-10, less than 1 / 256
+//   (the values of a unit) beside any weight.  On an x of size 1e-36: 5e-5 off 64 bits unscaled, 1e-7 scaled.  The test
+//   costs up to 0.2 us at 8 tokens (IQ4_XS 640 x 2560 6.45 / 6.66 us; one token 4.19 either way), the scaling nothing.
+//   Scaled under a branch instead, or split a second time where bits are lost, it cost 30 registers.
 template <uint32_t TY> struct MxX {
     static constexpr int MAP = MX<TY>::MAP, NS = MX<TY>::SUB ? 2 : 1;
     static constexpr bool MIN = MX<TY>::MIN, DEN = MX<TY>::DEN;
+    using Exp = std::conditional_t<DEN, int, uint64_t>;
     f4v a[2], b[2];
     __device__ __forceinline__ void load(const float *__restrict__ x, int cols, int u, int t0, int nt, int lane, bool single) {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
@@ -432,7 +444,30 @@ template <uint32_t TY> struct MxX {
         return s;
     }
     // x's scale: the largest magnitude (of the token's 256 values) to just under 2^120
-    static __device__ __forceinline__ int scale_of(float mx) { return min(246 - (int) (__float_as_uint(mx) >> 23), 126); }
+    static __device__ __forceinline__ int scale_of(float mx) { return 246 - (int) (__float_as_uint(mx) >> 23); }
+    static constexpr int UP = 53;
+    // test(): the lanes whose token's unit is scaled, by round.  A unit is not if a value is at least 2^-63 (its exponent's
+    // first or second bit is set), an infinity or a NaN.
+    uint64_t up[2];
+    __device__ __forceinline__ void test(int rounds, bool one) {
+        if constexpr (DEN) return;
+        const auto large = [](const f4v &c) {
+            return __float_as_uint(c[0]) | __float_as_uint(c[1]) | __float_as_uint(c[2]) | __float_as_uint(c[3]);
+        };
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if (r >= rounds) break;
+            const uint64_t big = __ballot(((one ? large(a[0]) : large(a[r]) | large(b[r])) & 0x60000000u) != 0);
+            const uint32_t t0 = (uint32_t) big, t1 = (uint32_t) (big >> 32);
+            const uint32_t u0 = (one ? t0 | t1 : t0) ? 0u : ~0u, u1 = (one ? t0 | t1 : t1) ? 0u : ~0u;
+            up[r] = (uint64_t) u1 << 32 | u0;
+        }
+    }
+    template <int N> __device__ __forceinline__ void scale_up(int r, float *v) const {
+        const float sc = __builtin_amdgcn_inverse_ballot_w64(up[r]) ? __builtin_ldexpf(1.0f, UP) : 1.0f;
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] *= sc;
+    }
     static __device__ __forceinline__ void fence() {
         // (LDS operations of a wave are done in order; the fences keep the compiler to it)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -440,16 +475,17 @@ template <uint32_t TY> struct MxX {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     // split() of one token, the same bits with half the work a lane (mx_one)
-    __device__ __forceinline__ void split1(int lane, uint8_t *lds, v4u *f) const {
+    __device__ __forceinline__ void split1(int lane, uint8_t *lds, v4u *f, Exp &xexp) const {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
         float v[4] = {a[0][0], a[0][1], a[0][2], a[0][3]};
-        uint32_t h[4], m[4], l[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) split3(v[k], h[k], m[k], l[k]);
+        uint32_t h[2], m[2], l[2];
+        xexp = up[0];
+        scale_up<4>(0, v);
+        split_n<4>(v, h, m, l);
         v2u *dst = reinterpret_cast<v2u *>(lds + (gl * 4 + q) * 48 + 8 * ts);
-        dst[0] = v2u{pack_hi(h[0], h[1]), pack_hi(h[2], h[3])};
-        dst[2] = v2u{pack_hi(m[0], m[1]), pack_hi(m[2], m[3])};
-        dst[4] = v2u{pack_hi(l[0], l[1]), pack_hi(l[2], l[3])};
+        dst[0] = v2u{h[0], h[1]};
+        dst[2] = v2u{m[0], m[1]};
+        dst[4] = v2u{l[0], l[1]};
         fence();
         // (every row takes the one token: those of the others are not used)
         const uint8_t *src = lds + (lane >> 4) * 48 + 16 * min(lane & 3, 2);
@@ -457,9 +493,10 @@ template <uint32_t TY> struct MxX {
         for (int j = 0; j < 8; ++j) f[j] = *reinterpret_cast<const v4u *>(src + j * 4 * 48);
         fence();
     }
-    __device__ __forceinline__ void split(int rounds, int lane, uint8_t *lds, v4u *f, float *sums, int &xexp) const {
+    __device__ __forceinline__ void split(int rounds, int lane, uint8_t *lds, v4u *f, float *sums, Exp &xexp) const {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
         int *exps = reinterpret_cast<int *>(lds + MX_X);
+        if constexpr (!DEN) xexp = 0;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             if (r >= rounds) break;
@@ -486,15 +523,17 @@ template <uint32_t TY> struct MxX {
                 mx = row_max(mx);
                 mx = fmaxf(mx, swz_xor16(mx));  // over the token's 256 values
                 const int e = scale_of(mx);
-                const float sc = __uint_as_float((uint32_t) (e + 127) << 23);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) v[k] *= sc;
+                for (int k = 0; k < 8; ++k) v[k] = ldexpf(v[k], e);
                 if ((lane & 31) == 0) exps[ts] = e;
+            } else {
+                scale_up<8>(r, v);
+                xexp |= ((up[r] & 0xFFFFull) | ((up[r] >> 32) & 0xFFFFull) << 16) << (32 * r);
             }
-            v4u h, m, l;
-            split8(v, h, m, l);
+            uint32_t h[4], m[4], l[4];
+            split_n<8>(v, h, m, l);
             v4u *dst = reinterpret_cast<v4u *>(lds + ((ts * 8 + gl) * 4 + q) * 48);
-            dst[0] = h, dst[1] = m, dst[2] = l;
+            dst[0] = v4u{h[0], h[1], h[2], h[3]}, dst[1] = v4u{m[0], m[1], m[2], m[3]}, dst[2] = v4u{l[0], l[1], l[2], l[3]};
             fence();
             const int row = lane & 15, tk = row >> 2, part = min(row & 3, 2);
             if (r == 0 || (tk >> 1) == 1) {
@@ -521,7 +560,8 @@ __device__ __forceinline__ float mx_sum3(const f4v &d) { return d[0] + (d[1] + d
 
 // one unit's products (lane (r, c): weight row r, token c of each token tile); the groups' sums in two chains
 template <uint32_t TY, int NTILE>
-__device__ __forceinline__ void mx_unit(uint32_t *w, const v4u (&f)[NTILE][8], const float *sums, const int (&xexp)[NTILE], int lane, const uint8_t *tab, float *out) {
+__device__ __forceinline__ void mx_unit(uint32_t *w, const v4u (&f)[NTILE][8], const float *sums,
+                                        const typename MxX<TY>::Exp (&xexp)[NTILE], int lane, const uint8_t *tab, float *out) {
     using F = MX<TY>;
     const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
     float acc[NTILE][2], mins[NTILE][2];
@@ -567,11 +607,13 @@ __device__ __forceinline__ void mx_unit(uint32_t *w, const v4u (&f)[NTILE][8], c
 #pragma unroll
     for (int i = 0; i < NTILE; ++i) {
         float v = acc[i][0] + acc[i][1];
-        if constexpr (F::DEN) v = ldexpf(v, 133 - F::SHIFT - xexp[i]);
         if constexpr (F::MIN) {
             float d, dm;
             F::super(w, d, dm);
-            v = __builtin_fmaf(-dm, mins[i][0] + mins[i][1], d * v);
+            // (the power of two last: before d, a sum near fp32's smallest values would lose bits that d v has)
+            v = __builtin_fmaf(-dm, mins[i][0] + mins[i][1], ldexpf(d * v, 133 - F::SHIFT - xexp[i]));
+        } else {
+            v *= __builtin_amdgcn_inverse_ballot_w64(xexp[i]) ? __builtin_ldexpf(1.0f, -MxX<TY>::UP) : 1.0f;
         }
         out[i] += v;
     }
@@ -618,15 +660,17 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
     load(blk, 0, wa, true, false);
     mx_tab_fill<TY>(tab, tid, blockDim.x);
     v4u f[UPW][NTILE][8];
-    int xexp[UPW][NTILE];
+    typename MxX<TY>::Exp xexp[UPW][NTILE];
     const bool one = mx_one<TY>(NTILE) && nt - t0 == 1;
+    const auto rounds = [&](int i) { return nt - t0 - 4 * i > 2 ? 2 : 1; };
 #pragma unroll
     for (int k = 0; k < UPW; ++k)
 #pragma unroll
         for (int i = 0; i < NTILE; ++i) {
             float *s = sums + (k * NTILE + i) * SUMS;
-            if (one) xr[k][i].split1(lane, mine, f[k][i]);
-            else xr[k][i].split(nt - t0 - 4 * i > 2 ? 2 : 1, lane, mine, f[k][i], s, xexp[k][i]);
+            xr[k][i].test(rounds(i), one);
+            if (one) xr[k][i].split1(lane, mine, f[k][i], xexp[k][i]);
+            else xr[k][i].split(rounds(i), lane, mine, f[k][i], s, xexp[k][i]);
         }
     if constexpr (HALF) load(blk, 0, wa, false, true);
     if constexpr (UPW == 2) load(blk, 1, wb);

@@ -407,3 +407,30 @@ def test_gemv_matrix_cores_short_second_tile(fnlib, name):
     y = fnlib.gemv(t, raw, rows, cols, x)
     for nt in (5, 6, 7):
         assert np.array_equal(fnlib.gemv(t, raw, rows, cols, x[:nt]).view(np.uint32), y[:nt].view(np.uint32)), nt
+
+
+@pytest.mark.parametrize("name", MX_TYPES)
+@pytest.mark.parametrize("nt", [1, 8])
+def test_gemv_matrix_cores_small_x(fnlib, name, nt):
+    """An x near the end of fp32's range (bf16's smallest value is 2^-133, so its low bits have no bf16 as they stand)
+    keeps its 24 bits, in rows of one and of two units a wave.  Bound: as test_gemv_matrix_cores, and the roundings at
+    fp32's smallest value that a result below 2^-126 has: one a unit and one a sum."""
+    t, rows = TYPES[name], 20
+    _say(f"gemv matrix cores, small x, {name} nt={nt}")
+    for cols in (2560, 4608):
+        rng = np.random.default_rng(13)
+        raw = random_finite(t, rows, cols, rng)
+        if name == "BF16":
+            raw = (rng.standard_normal(rows * cols).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).view(np.uint8)
+        else:
+            blk = raw.reshape(-1, oracle.qblock(t)[1])
+            for b in {8: [1], 20: [1], 21: [1], 23: [1], 12: [1, 3], 13: [1, 3], 14: [209]}[t]:
+                blk[:, b] = 0x40                     # scales of 2 to 3: results of the size of x and larger
+        x = rng.standard_normal((8, cols))
+        for size in (1e-32, 1e-34, 1e-36, 1e-38, 1e-40):
+            xs = (x * size).astype(np.float32)
+            ref = oracle.gemv(t, raw, rows, cols, xs)
+            for i in range(8 // nt):
+                y = fnlib.gemv(t, raw, rows, cols, xs[i * nt:(i + 1) * nt])
+                tol = 2e-6 * np.abs(ref).max() + 2 * (cols // 256) * 2.0 ** -149
+                assert np.abs(y - ref[i * nt:(i + 1) * nt]).max() <= tol, (cols, size, i)
