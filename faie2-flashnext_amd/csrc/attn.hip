@@ -624,8 +624,9 @@ __device__ __forceinline__ void mt_walk(const float4 *Kb, const float4 *Vb, cons
 
 // grid (nsplit, nkv, B), RW * KW <= 4 waves; dynamic LDS: max(RW * NRW * 16 KiB of Q, RW * KW * 16 * MT_OS * 4 B), MX:
 // 24 KiB of Q a row block; KEEP = RW > 1 (row groups share each block through the L2)
-// MX: the walk on the bf16 matrix cores (attn_mx.cuh); a split whose sums hold a NaN is walked again in fp32, so that
-// infinities and NaN in the inputs give what the fp32 walk gives.
+// MX: the walk on the bf16 matrix cores (attn_mx.cuh); a split that the bf16 parts do not hold is walked in fp32: instead,
+// if a query element is out of their range; again, if a merged sum is.  Infinities, NaN and values near the ends of fp32's
+// range so give what the fp32 walk gives.
 template <int NRW, bool KEEP, bool MX>
 __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
@@ -668,6 +669,7 @@ k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
         }
     };
     reset();
+    bool f32 = !MX;  // the walk is (to be) the fp32 one
     auto walk_f32 = [&]() {
         // Q of all row blocks into LDS: [row block][u][lane] float4, lane l = (row l%16, chunk 4u + l/16)
         for (int i = tid; i < RW * NRW * 1024; i += nth)
@@ -691,6 +693,7 @@ k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
     if constexpr (MX) {
         // Q in parts: [row block][u][part][lane] of 8 bf16, lane l = (row l%16, chunks 8u + l/16 and 8u + 4 + l/16)
         v4u *qd = reinterpret_cast<v4u *>(mt_lds);
+        MxRange seen;
         for (int i = tid; i < RW * NRW * 512; i += nth) {
             const int rb = i >> 9, u = (i >> 6) & 7, ln = i & 63, row = rb * 16 + (ln & 15), c = 8 * u + (ln >> 4);
             const float4 x0 = q_chunk(row, c), x1 = q_chunk(row, c + 4);
@@ -698,13 +701,14 @@ k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
             Mx3 d;
             mx_split(x, d);
 #pragma unroll
+            for (int k = 0; k < 8; ++k) seen.see(x[k]);
+#pragma unroll
             for (int p = 0; p < 3; ++p) qd[rb * MX_QB + (u * 3 + p) * 64 + ln] = d.p[p];
         }
-        __syncthreads();
+        f32 = __syncthreads_or(seen.out<-110, 90>());
         const int nblk = k1 > k0 ? (k1 - k0 + 31) / 32 : 0;
         const int nw = nblk > kw ? (nblk - 1 - kw) / KW + 1 : 0;  // this wave's blocks of 32 keys
-        bool bad = false;
-        if (nw > 0) {
+        if (nw > 0 && !f32) {
             MxWalk<KEEP> w;
             w.Kb = reinterpret_cast<const char *>(Kb), w.Vb = reinterpret_cast<const char *>(Vb);
             w.qs = qd + rw * NRW * MX_QB;
@@ -719,74 +723,76 @@ k_attn_split_mt(const AttnArgs a, int grp, int RW, int KW) {
 #pragma unroll
             for (int j = 0; j < NRW; ++j) {
                 m[j] = w.m[j], l[j] = w.l[j];
-                float s = l[j];
 #pragma unroll
-                for (int t2 = 0; t2 < 16; ++t2) {
-                    o[j][t2] = w.o[j][t2];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s = fmaf(o[j][t2][r], 0.0f, s);  // an infinity becomes a NaN too
-                }
-                bad |= s != s;
+                for (int t2 = 0; t2 < 16; ++t2) o[j][t2] = w.o[j][t2];
             }
         }
-        if (__syncthreads_or(bad)) {
-            reset();
+    }
+    for (;;) {
+        if (f32) {
+            if (MX) reset();
             walk_f32();
         }
-    } else {
-        walk_f32();
-    }
 
-    // merge the KW key streams of each row group (log-sum-exp), then write the split partials
+        // merge the KW key streams of each row group (log-sum-exp), then write the split partials
 #pragma unroll
-    for (int j = 0; j < NRW; ++j) {
-        l[j] = sum_x16_x32(l[j]);
-        if (lane < 16) mls[wave][j * 16 + lane] = make_float2(m[j], l[j]);
-    }
-    __syncthreads();  // Q is dead: the LDS becomes the merge buffer
-    float *ob = reinterpret_cast<float *>(mt_lds);
-#pragma unroll
-    for (int j = 0; j < NRW; ++j) {
-        {
-            const int row = lane & 15;
-            float M = -INFINITY;
-            for (int w = 0; w < KW; ++w) M = fmaxf(M, mls[rw * KW + w][j * 16 + row].x);
-            const float sc = m[j] == -INFINITY ? 0.0f : expf(m[j] - M);
-            float *dst = ob + (wave * 16 + row) * MT_OS + 16 * (lane >> 4);
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    *reinterpret_cast<float4 *>(dst + 64 * c + 4 * q) =
-                        make_float4(o[j][4 * c][q] * sc, o[j][4 * c + 1][q] * sc, o[j][4 * c + 2][q] * sc,
-                                    o[j][4 * c + 3][q] * sc);
+        for (int j = 0; j < NRW; ++j) {
+            l[j] = sum_x16_x32(l[j]);
+            if (lane < 16) mls[wave][j * 16 + lane] = make_float2(m[j], l[j]);
         }
-        __syncthreads();
-        for (int i = tid; i < RW * 16 * 64; i += nth) {
-            const int rg = i >> 10, row = (i >> 6) & 15, d4 = i & 63;
-            const int rowg = (rg * NRW + j) * 16 + row;
-            if (rowg < R) {
-                float4 O = f4(0.0f);
-                for (int w = 0; w < KW; ++w) {
-                    const float4 x = *reinterpret_cast<const float4 *>(ob + ((rg * KW + w) * 16 + row) * MT_OS + 4 * d4);
-                    O.x += x.x; O.y += x.y; O.z += x.z; O.w += x.w;
-                }
-                const int t = rowg / grp, h = rowg - t * grp;
-                const size_t pi = ((size_t) (b * a.nt + t) * a.nq + g * grp + h) * a.nsplit + sp_i;
-                reinterpret_cast<float4 *>(a.part_o + pi * HD)[d4] = O;
-                if (d4 == 0) {
-                    float M = -INFINITY, L = 0.0f;
-                    for (int w = 0; w < KW; ++w) M = fmaxf(M, mls[rg * KW + w][j * 16 + row].x);
+        __syncthreads();  // Q is dead: the LDS becomes the merge buffer
+        float *ob = reinterpret_cast<float *>(mt_lds);
+        const float osc = MX && !f32 ? 1.0f / MX_PUP : 1.0f;
+        MxRange seen;
+#pragma unroll
+        for (int j = 0; j < NRW; ++j) {
+            {
+                const int row = lane & 15;
+                float M = -INFINITY;
+                for (int w = 0; w < KW; ++w) M = fmaxf(M, mls[rw * KW + w][j * 16 + row].x);
+                const float sc = m[j] == -INFINITY ? 0.0f : expf(m[j] - M);
+                float *dst = ob + (wave * 16 + row) * MT_OS + 16 * (lane >> 4);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<float4 *>(dst + 64 * c + 4 * q) =
+                            make_float4(o[j][4 * c][q] * sc, o[j][4 * c + 1][q] * sc, o[j][4 * c + 2][q] * sc,
+                                        o[j][4 * c + 3][q] * sc);
+            }
+            __syncthreads();
+            for (int i = tid; i < RW * 16 * 64; i += nth) {
+                const int rg = i >> 10, row = (i >> 6) & 15, d4 = i & 63;
+                const int rowg = (rg * NRW + j) * 16 + row;
+                if (rowg < R) {
+                    float4 O = f4(0.0f);
                     for (int w = 0; w < KW; ++w) {
-                        const float2 ml = mls[rg * KW + w][j * 16 + row];
-                        if (ml.x != -INFINITY) L = fmaf(expf(ml.x - M), ml.y, L);
+                        const float4 x = *reinterpret_cast<const float4 *>(ob + ((rg * KW + w) * 16 + row) * MT_OS + 4 * d4);
+                        O.x += x.x; O.y += x.y; O.z += x.z; O.w += x.w;
                     }
-                    a.part_ml[pi * 2] = M;
-                    a.part_ml[pi * 2 + 1] = L;
+                    if constexpr (MX) {
+                        seen.see(O.x), seen.see(O.y), seen.see(O.z), seen.see(O.w);
+                        O.x *= osc, O.y *= osc, O.z *= osc, O.w *= osc;
+                    }
+                    const int t = rowg / grp, h = rowg - t * grp;
+                    const size_t pi = ((size_t) (b * a.nt + t) * a.nq + g * grp + h) * a.nsplit + sp_i;
+                    reinterpret_cast<float4 *>(a.part_o + pi * HD)[d4] = O;
+                    if (d4 == 0) {
+                        float M = -INFINITY, L = 0.0f;
+                        for (int w = 0; w < KW; ++w) M = fmaxf(M, mls[rg * KW + w][j * 16 + row].x);
+                        for (int w = 0; w < KW; ++w) {
+                            const float2 ml = mls[rg * KW + w][j * 16 + row];
+                            if (ml.x != -INFINITY) L = fmaf(expf(ml.x - M), ml.y, L);
+                        }
+                        a.part_ml[pi * 2] = M;
+                        a.part_ml[pi * 2 + 1] = L;
+                    }
                 }
             }
+            if (j + 1 < NRW) __syncthreads();
         }
-        __syncthreads();
+        if (!MX || f32 || !__syncthreads_or(seen.out<-56, 128>())) break;
+        f32 = true;
     }
 }
 

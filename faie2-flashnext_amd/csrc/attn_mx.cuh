@@ -29,6 +29,28 @@ constexpr int MX_NRW = 2;                       // 16-row blocks a wave
 constexpr int MX_QB = 8 * 3 * 64;               // 16-byte Q fragments of a 16-row block: [u][part][lane]
 constexpr int MX_MAXCTX = 1 << 21;              // 32-bit byte offsets into a head's cache
 
+// What three bf16 parts hold: a value from 2^-110 on exactly, a smaller one to 2^-134 (bf16 has nothing below 2^-133).
+//   P: a probability is 0 or at least fp32's smallest normal number, 2^-126, so its parts are those of MX_PUP p; the
+//     sums over V come out scaled by it.
+//   Q: an element other than 0 must not be too small, nor so large (2^90) that what K's small elements lose would count in
+//     the score (at most 2^-134 2^90 a term).
+//   V: what it loses counts only in a small sum: a value loses at most 2^-134, beside a probability of at most 2^28
+//     (MX_PUP e^MT_SLACK) and 2^21 keys 2^-85 in all, and products that underflow lose less; so a sum of the split, over
+//     its streams, must be 2^-56 or larger, or 0 (rows that see no key, dims that hold none), and finite.  (Looked at in
+//     the merge and not in the walk's registers, where it cost 2 us: 128 sums a lane of code that runs once.)
+constexpr float MX_PUP = 65536.0f;
+struct MxRange {  // the least and largest magnitudes seen other than 0, as bits from bit 1 (least: less 1)
+    uint32_t least = ~0u, most = 0u;
+    __device__ __forceinline__ void see(float x) {
+        const uint32_t u = __float_as_uint(x) << 1;
+        least = min(least, u - 1);
+        most = max(most, u);
+    }
+    template <int LO, int HI> __device__ __forceinline__ bool out() const {  // below 2^LO, or 2^HI or larger, or a NaN
+        return least < ((127u + LO) << 24) - 1 || most >= (127u + HI) << 24;
+    }
+};
+
 struct Mx3 {  // 8 values a lane, in three bf16 parts
     v4u p[3];
 };
@@ -37,7 +59,7 @@ __device__ __forceinline__ uint32_t mx_cvt(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), bf16x2));
 }
 // part PH of values 2k, 2k + 1 of x; r holds their remainder between the parts.  An infinity or NaN (or a value that
-// rounds to infinity) leaves a NaN in a later part, which mx_walk's caller finds in the sums.
+// rounds to infinity) leaves a NaN in a later part, which is found in the sums.
 __device__ __forceinline__ void mx_split_piece(int k, int ph, const float (&x)[8], float (&r)[2], Mx3 &d) {
     const float a = ph == 0 ? x[2 * k] : r[0], b = ph == 0 ? x[2 * k + 1] : r[1];
     const uint32_t h = mx_cvt(a, b);
@@ -196,6 +218,8 @@ struct MxWalk {
             }
             l[j] = fmaf(l[j], corr[j], ps);
             m[j] = mn;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[i] *= MX_PUP;
             mx_split(p, P[j]);
         }
         mt_rescale<MX_NRW>(o, corr);

@@ -265,3 +265,58 @@ def test_attn_position_outside_cache_sets_status(fnlib):
         assert K.download().shape == k0.shape and V.download().shape == v0.shape
         for x in (K, V, work, og, *d.values()):
             x.free()
+
+
+@pytest.mark.parametrize("nq,nt", [(16, 3), (16, 8), (24, 8)])
+@pytest.mark.parametrize("size", [1e-19, 1e-34, 1e-36, 1e-38])
+def test_attn_multi_token_small_values(fnlib, nq, nt, size):
+    """Cached and new values near the end of fp32's range keep their bits, where bf16 (smallest value 2^-133) does not
+    hold them as three parts; the last token's value is of size 1, which the tokens before it do not see.  Bound: that
+    of test_attn_bf16_parts_walk, token by token."""
+    _say(f"attn multi-token small values nq={nq} nt={nt} size={size}")
+    case = _mt_case(2, nq, 2, nt, [300, 129], 512, seed=3 + nt)
+    for a in (case.Vc, case.v[:, :-1]):
+        a[:] = (a.astype(np.float64) * size).astype(np.float32)
+    og = fnlib.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc.copy(), case.Vc.copy(), case.pos)
+    ref, _, _ = oracle.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc, case.Vc, case.pos)
+    og, ref = (np.asarray(a, np.float64).reshape(2, nt, -1) for a in (og, ref))
+    for t in range(nt):
+        scale = np.abs(ref[:, t]).max()
+        assert np.linalg.norm((og[:, t] - ref[:, t]) / scale) <= 2e-6 * np.linalg.norm(ref[:, t] / scale), t
+
+
+@pytest.mark.parametrize("nq,nt", [(16, 4), (24, 8)])
+def test_attn_multi_token_small_probability(fnlib, nq, nt):
+    """A key of probability 2^-122 whose value, 1e38 times the others', makes most of the result.  Bound: the exponent
+    of that probability has 24 bits at a size of 122, so 122 * 2^-24 in the probability (7e-6), and twice that for the
+    score (85, from 192 terms) and the scale of the softmax."""
+    _say(f"attn multi-token small probability nq={nq} nt={nt}")
+    case = _mt_case(1, nq, 2, nt, [200], 256, seed=9)
+    case.qg[..., 0, :] = case.qg[0, 0, 0, 0]                     # one query row, the same at every position in
+    q = case.qg[0, 0, 0, 0].astype(np.float64)                   # the dims past the rotated ones
+    q = q / np.sqrt((q * q).mean() + 1e-6) * case.wq
+    q[:64] = 0.0
+    case.Kc[:] = 0.0
+    case.Kc[0, 77] = (-85.0 * 16.0 * q / (q * q).sum()).astype(np.float32)
+    case.k[..., 64:] *= np.float32(1e-3)                         # (new keys: scores near 0)
+    case.Vc[:] *= np.float32(1e-8)
+    case.v[:] *= np.float32(1e-8)
+    case.Vc[0, 77] = np.float32(1e30) * np.sign(case.Vc[0, 77])
+    og = fnlib.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc.copy(), case.Vc.copy(), case.pos)
+    ref, _, _ = oracle.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc, case.Vc, case.pos)
+    assert oracle.relerr(og, ref) <= 2.5e-5
+
+
+@pytest.mark.parametrize("nq,nt", [(16, 4), (24, 8)])
+def test_attn_multi_token_query_out_of_range(fnlib, nq, nt):
+    """Query rows of size 1e-36 (a tiny norm weight) over keys of size 1e36, and the other way round: the scores, of
+    size 1, keep fp32's precision."""
+    for wq, key in ((1e-36, 1e36), (1e36, 1e-36)):
+        _say(f"attn multi-token query out of range nq={nq} nt={nt} wq={wq}")
+        case = _mt_case(2, nq, 2, nt, [300, 129], 512, seed=21)
+        case.wq[:] *= np.float32(wq)
+        case.wk[:] *= np.float32(key)
+        case.Kc[:] *= np.float32(key)
+        og = fnlib.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc.copy(), case.Vc.copy(), case.pos)
+        ref, _, _ = oracle.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc, case.Vc, case.pos)
+        assert oracle.relerr(og, ref) <= 2e-6
