@@ -115,7 +115,8 @@ __global__ void __launch_bounds__(256) k_ix_prep(const IxArgs a) {
     }
     __syncthreads();  // the raw keys written above are read back below
     const int end = min(pos + a.nt, a.max_ctx);
-    for (int j = pos / IXR + wave; j < end / IXR; j += 4) block_key(a, b, j, buf[wave], lane);
+    if (pos >= 0)  // (nothing was appended to a call that starts before the cache, and its blocks would too)
+        for (int j = pos / IXR + wave; j < end / IXR; j += 4) block_key(a, b, j, buf[wave], lane);
 }
 
 // grid (B, ceil((j1 - j0) / 4)), 256 threads: block keys of blocks [j0, j1) of every sequence
@@ -165,8 +166,9 @@ __global__ void __launch_bounds__(256) k_ix_score(const IxArgs a, const AT at) {
     const int ntiles = (nb + BT - 1) / BT;
     int tile = blockIdx.y;
     const bool live = nb > a.top && tile < ntiles;  // sparse query, and this workgroup has tiles
-    const int jnew = max(pos, 0) / IXR, jw = jnew + (ATTN ? wave : 0);
-    // PREP: blocks jnew .. nb - 1 are new (one token: at most one, wave 0's), block jw is this wave's
+    const int jnew = pos >= 0 ? pos / IXR : a.max_ctx / IXR, jw = jnew + (ATTN ? wave : 0);
+    // PREP: blocks jnew .. nb - 1 are new (one token: at most one, wave 0's; none of a call that starts before the cache:
+    // nothing of it is appended), block jw is this wave's
     // PREP: the head's query row, the new raw key and the raw keys of the wave's new block requested first
     // (unconditional, clamped), so that the query's norm and RoPE wait for them and not for the tile
     float2 x, nk, rk[IXR];
@@ -192,8 +194,8 @@ __global__ void __launch_bounds__(256) k_ix_score(const IxArgs a, const AT at) {
         for (int c = 0; c < CW; ++c) kf[c] = ld_nt(&Bb[((size_t) tile * (IXD / 4) + c) * BT]);
     }
     if constexpr (PREP) {
-        const bool valid = P >= 0 && P < a.max_ctx;
-        if (!valid) {  // past the cache: nothing to append; the status word says so
+        const bool valid = pos >= 0 && P < a.max_ctx;
+        if (!valid) {  // outside the cache: nothing to append; the status word says so
             if (blockIdx.y == 0 && threadIdx.x == 0) atomicOr(a.status, FN_STATUS_POS);
         } else if (blockIdx.y == 0 && wave == 0) {
             reinterpret_cast<float2 *>(a.IKc + ((size_t) b * a.max_ctx + P) * IXD)[lane] = nk;

@@ -343,3 +343,43 @@ def test_qsa_prep_folded_same_bits(fnlib, pos):
     assert (fnlib.dev_status() != 0) == (max(pos) + 17 > max_ctx)
     for b in w.values():
         b.free()
+
+
+@pytest.mark.parametrize("nt,p0", [(1, -1), (4, -2), (16, -2), (17, -2), (17, -5)])
+def test_qsa_call_starting_before_the_cache(fnlib, nt, p0):
+    """A call that starts at a negative position appends nothing to the indexer's caches, on every path (its prep in
+    the scoring launch or in one of its own): the raw and block keys stay as they were, the status bit is set, and the
+    other sequence's keys are appended."""
+    import fn
+
+    _say(f"qsa call starting before the cache nt={nt} pos={p0}")
+    B, nq, nkv, hd, max_ctx, top = 2, 16, 2, 256, 512, 32
+    fnlib.dev_status()  # start clean
+    rng = np.random.default_rng(15)
+    nsplit = 2
+    wb = fnlib.attn_qsa_work_bytes(B, nq, nt, nsplit, max_ctx, top)
+    cache = B * nkv * max_ctx * hd
+    d = {n: hiprt.Buf.empty((m,)) for n, m in (("K", cache), ("V", cache), ("IK", B * max_ctx * 128),
+                                               ("BK", B * max_ctx // 4 * 128))}
+    for j, buf in enumerate(d.values()):
+        fnlib.fill_normal_dev(buf.ptr, buf.nbytes // 4, 80 + j)
+    hiprt.sync()
+    ik0, bk0 = d["IK"].download((B, max_ctx, 128)), d["BK"].download((B, max_ctx // 4 * 128))
+    iqk = rng.standard_normal((B, nt, 640)).astype(np.float32)
+    d |= {n: hiprt.Buf.like(x) for n, x in (
+        ("qg", rng.standard_normal((B, nt, nq, 2, hd)).astype(np.float32)),
+        ("k", rng.standard_normal((B, nt, nkv, hd)).astype(np.float32)),
+        ("v", rng.standard_normal((B, nt, nkv, hd)).astype(np.float32)), ("iqk", iqk),
+        ("wq", np.ones(hd, np.float32)), ("wk", np.ones(hd, np.float32)), ("wqn", np.ones(128, np.float32)),
+        ("wkn", np.ones(128, np.float32)), ("pos", np.array([p0, 300], np.int32)))}
+    work, og = hiprt.Buf(wb), hiprt.Buf.empty((B, nt, nq, hd))
+    work.zero()
+    fnlib.attn_qsa_dev(B, nq, nkv, nt, max_ctx, d["pos"].ptr, d["qg"].ptr, d["k"].ptr, d["v"].ptr, d["wq"].ptr,
+                       d["wk"].ptr, d["K"].ptr, d["V"].ptr, d["iqk"].ptr, d["wqn"].ptr, d["wkn"].ptr, d["IK"].ptr,
+                       d["BK"].ptr, top, nsplit, work.ptr, wb, og.ptr)
+    assert fnlib.dev_status() == fn.STATUS_POS
+    ik, bk = d["IK"].download((B, max_ctx, 128)), d["BK"].download((B, max_ctx // 4 * 128))
+    assert np.array_equal(ik[0], ik0[0]) and np.array_equal(bk[0], bk0[0])
+    assert np.array_equal(ik[1, 300:300 + nt], iqk[1, :, 512:]) and np.array_equal(ik[1, :300], ik0[1, :300])
+    for x in (work, og, *d.values()):
+        x.free()
