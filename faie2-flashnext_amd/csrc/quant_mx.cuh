@@ -799,6 +799,7 @@ int mx_launch(const QLayout &L, const uint8_t *packed, const float *x, int nt, f
     const int halves = (nt + 4 * NTILE - 1) / (4 * NTILE), ntiles = (L.rows + rt - 1) / rt;
     int per_cu = 0;
     if (mx_per_cu(k_gemv_mx<TY, NTILE, UPW, MAXT>, cache, W, lds, per_cu)) return -1;
+    if (g_ov_wpc) per_cu = std::max(1, g_ov_wpc / W);
     const int nwg = g_persist ? std::min(ntiles, std::max(1, device_cus() * per_cu / halves)) : ntiles;
     hipLaunchKernelGGL((k_gemv_mx<TY, NTILE, UPW, MAXT>), dim3((unsigned) nwg, (unsigned) halves), dim3(64 * W), (size_t) lds,
                        st, planes(L, packed), L.rows, rt, U, x, L.cols, nt, y);

@@ -52,10 +52,10 @@ int fn_test_dequant(uint32_t type, const uint8_t *W, int rows, int cols, float *
  * ks: split-K workgroups per row, as the reference's (out[2]).  tb: not the reference's tiles per block (the
  * workgroups here are fixed at 8 waves) but this library's kernel choice (1 x staged in chunks, 2 x staged once,
  * 3 / 4 x staged once with the deep / short walk).  warps_per_sm: the resident waves per CU a persistent grid is
- * sized for (the reference's target warps per SM).  A forced wpt, ks > 1 or tb takes the vector kernels; without one,
- * most shapes run on the matrix cores, which sum in an order of their own (the same to about 1e-7).  Lanes per row and
- * ks > 1 change the summation order, the other choices give the same bits among themselves.  The model forward's GEMVs
- * take no split-K whatever ks asks (no work buffer). */
+ * sized for (the reference's target warps per SM), on either kind of kernel; it changes neither path nor bits.  A
+ * forced wpt, ks > 1 or tb takes the vector kernels; without one, most shapes run on the matrix cores, which sum in an
+ * order of their own (the same to about 1e-7).  Lanes per row and ks > 1 change the summation order, the other choices
+ * give the same bits among themselves.  The model forward's GEMVs take no split-K whatever ks asks (no work buffer). */
 void fn_gemv_override(int wpt, int ks, int tb, int warps_per_sm);             /* faie2fn.cu:2786 */
 /* The reference's persistent-grid switch: waves != 0 (default) launches the GEMV on the workgroups resident at once,
  * each walking many row tiles; 0 launches one workgroup per row tile.  Same bits either way; fn_gemv_plan's out[5]

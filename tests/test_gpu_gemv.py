@@ -10,6 +10,8 @@ real tensors are not in this image).
 Every case prints what names it before the GPU call.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -434,3 +436,47 @@ def test_gemv_matrix_cores_small_x(fnlib, name, nt):
                 y = fnlib.gemv(t, raw, rows, cols, xs[i * nt:(i + 1) * nt])
                 tol = 2e-6 * np.abs(ref).max() + 2 * (cols // 256) * 2.0 ** -149
                 assert np.abs(y - ref[i * nt:(i + 1) * nt]).max() <= tol, (cols, size, i)
+
+
+def _grid_of(fnlib, fn_call):
+    """grid of the one kernel that fn_call(stream) launches, from the graph that captures it"""
+    class Params(ctypes.Structure):
+        _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                    ("grid", ctypes.c_uint32 * 3), ("args", ctypes.c_void_p), ("lds", ctypes.c_uint32)]
+
+    st = hiprt.Stream()
+    g = hiprt.Graph(st, lambda: fn_call(st.handle))
+    n = ctypes.c_size_t(1)
+    node, p = ctypes.c_void_p(), Params()
+    hiprt.check(hiprt.lib().hipGraphGetNodes(ctypes.c_void_p(g.graph), ctypes.byref(node), ctypes.byref(n)), "nodes")
+    assert n.value == 1
+    hiprt.check(hiprt.lib().hipGraphKernelNodeGetParams(node, ctypes.byref(p)), "kernel node")
+    g.destroy()
+    st.destroy()
+    return tuple(p.grid)
+
+
+def test_gemv_matrix_cores_waves_per_cu(fnlib):
+    """The resident waves per CU that a persistent grid is sized for (fn_gemv_override's last argument), forced alone,
+    change the grid of a matrix-core launch and not its bits: 10 waves a workgroup here, 1250 tiles."""
+    t, rows, cols, nt = TYPES["Q5_K"], 20000, 2560, 3
+    _say(f"gemv matrix cores, forced waves per CU, Q5_K {rows}x{cols} nt={nt}")
+    raw = random_finite(t, rows, cols, RNG)
+    x = RNG.standard_normal((nt, cols)).astype(np.float32)
+    draw, dx = hiprt.Buf.like(raw), hiprt.Buf.like(x)
+    packed, dy = hiprt.Buf(fnlib.gemv_packed_bytes(t, rows, cols), np.uint8), hiprt.Buf.empty((nt, rows))
+    fnlib.gemv_pack_dev(t, draw.ptr, rows, cols, packed.ptr)
+    hiprt.sync()
+    y, grid = {}, {}
+    try:
+        for wpc in (0, 4, 10, 30):
+            fnlib.gemv_override(waves_per_cu=wpc)
+            grid[wpc] = _grid_of(fnlib, lambda st: fnlib.gemv_dev(t, packed.ptr, rows, cols, dx.ptr, nt, dy.ptr, None,
+                                                                  0, st))[0]
+            y[wpc] = fnlib.gemv(t, raw, rows, cols, x)
+    finally:
+        fnlib.gemv_override(0)
+    cus = grid[10]  # one workgroup a CU
+    assert 1 < cus <= 416 and grid[4] == cus and grid[30] == 3 * cus and grid[0] >= cus, grid
+    for wpc in (4, 10, 30):
+        assert np.array_equal(y[wpc], y[0]), wpc
