@@ -30,6 +30,9 @@
 //   BF16      96 x 2560     4.6 /  4.2    6.0 /  4.8    8.6 /   5.8
 //   Q4_K   20000 x 8192    27.4 / 22.8   47.9 / 24.3  124.0 /  33.5
 //   Q5_K  248320 x 2560   104.8 / 98.9  183.4 / 105.0  291.3 / 139.6
+//   Q5_K    2560 x 8192     9.8 /  8.9   14.1 / 11.2   28.6 /  16.3
+//   Q6_K   20000 x 8192    30.5 / 33.6   51.1 / 36.4  130.5 /  58.1
+//   Q6_K     300 x 8192     6.5 /  7.4    9.8 /  9.5   19.3 /   9.6
 //   grouped: DeltaNet's qkv, z (Q6_K), alpha and beta  12.4 / 11.4   23.0 / 12.6   32.8 / 16.3
 //            attention's q, k, v and indexer           12.0 / 10.6   19.4 / 11.3   27.4 / 14.8
 //            the FFN's router, shared gate and up       5.2 /  5.4    6.7 /  6.4    9.2 /   7.5
@@ -362,14 +365,21 @@ template <uint32_t TY> __device__ __forceinline__ void mx_tab_fill(uint8_t *tab,
 
 // LDS of a workgroup of W waves: the format's table, a piece a wave for the x split (64 fragments of 8 values x 3 parts,
 // the group sums, the exponents), two buffers of 16 waves' partial sums
-constexpr int MX_X = 64 * 48;
+constexpr int MX_X = 64 * 48, MX_GRP = 4 * 48;
 // (the sums of x of a token tile: 4 tokens x 8 groups, twice that for SUB; the formats without a minimum leave them out)
 constexpr int mx_sums(bool min, bool sub) { return min ? (sub ? 256 : 128) : 0; }
-template <uint32_t TY> constexpr int mx_wave(int upw, int ntile) {
-    return MX_X + 64 + upw * ntile * mx_sums(MX<TY>::MIN, MX<TY>::SUB);
+// Whether the second of a wave's two units keeps its split x in LDS, where every tile reads it again: where the 128 VGPRs of
+// a workgroup of 1024 threads do not hold two units of x, their words and the sums of x.  In registers Q5_K and Q6_K
+// spilled 41 and 34 (20000 x 8192, one token, 46.2 / 46.5 us; so 30.5 / 33.6); where two fit, LDS is slower (IQ4_XS 2560 x
+// 8192 8.0 / 8.4 us, and 9.6 instead of 8.3 for two tokens).
+template <uint32_t TY> constexpr bool mx_stay(int upw, int maxt) {
+    return upw == 2 && maxt == 1024 && MX<TY>::MIN && MX<TY>::NW >= 15;
 }
-template <uint32_t TY> constexpr int mx_lds(int W, int upw, int ntile) {
-    return mx_tab_bytes<TY>() + W * mx_wave<TY>(upw, ntile) + 2 * 16 * ntile * 256;
+template <uint32_t TY> constexpr int mx_wave(int upw, int ntile, int maxt) {  // (STAY: a piece for each of the two rounds)
+    return (mx_stay<TY>(upw, maxt) ? 2 : 1) * MX_X + 64 + upw * ntile * mx_sums(MX<TY>::MIN, MX<TY>::SUB);
+}
+template <uint32_t TY> constexpr int mx_lds(int W, int upw, int ntile, int maxt) {
+    return mx_tab_bytes<TY>() + W * mx_wave<TY>(upw, ntile, maxt) + 2 * 16 * ntile * 256;
 }
 
 // x = hi + mid + lo, each in the high 16 bits of a float: exact from |x| = 2^-110 on, where lo's low bits are zero by
@@ -474,6 +484,11 @@ template <uint32_t TY> struct MxX {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+    // where a lane's operand of group 0 is after a split() of that many rounds that stays in LDS
+    static __device__ __forceinline__ int piece(int rounds, int lane) {
+        const int row = lane & 15, tk = row >> 2, part = min(row & 3, 2);
+        return (rounds > 1 ? (tk >> 1) * MX_X : 0) + ((tk & 1) * 32 + (lane >> 4)) * 48 + 16 * part;
+    }
     // split() of one token, the same bits with half the work a lane (mx_one)
     __device__ __forceinline__ void split1(int lane, uint8_t *lds, v4u *f, Exp &xexp) const {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
@@ -487,15 +502,13 @@ template <uint32_t TY> struct MxX {
         dst[2] = v2u{m[0], m[1]};
         dst[4] = v2u{l[0], l[1]};
         fence();
-        // (every row takes the one token: those of the others are not used)
         const uint8_t *src = lds + (lane >> 4) * 48 + 16 * min(lane & 3, 2);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = *reinterpret_cast<const v4u *>(src + j * 4 * 48);
+        for (int j = 0; j < 8; ++j) f[j] = *reinterpret_cast<const v4u *>(src + j * MX_GRP);
         fence();
     }
-    __device__ __forceinline__ void split(int rounds, int lane, uint8_t *lds, v4u *f, float *sums, Exp &xexp) const {
+    __device__ __forceinline__ void split(bool stay, int rounds, int lane, uint8_t *lds, v4u *f, int *exps, float *sums, Exp &xexp) const {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
-        int *exps = reinterpret_cast<int *>(lds + MX_X);
         if constexpr (!DEN) xexp = 0;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
@@ -532,14 +545,14 @@ template <uint32_t TY> struct MxX {
             }
             uint32_t h[4], m[4], l[4];
             split_n<8>(v, h, m, l);
-            v4u *dst = reinterpret_cast<v4u *>(lds + ((ts * 8 + gl) * 4 + q) * 48);
+            v4u *dst = reinterpret_cast<v4u *>(lds + (stay ? r * MX_X : 0) + ((ts * 8 + gl) * 4 + q) * 48);
             dst[0] = v4u{h[0], h[1], h[2], h[3]}, dst[1] = v4u{m[0], m[1], m[2], m[3]}, dst[2] = v4u{l[0], l[1], l[2], l[3]};
             fence();
             const int row = lane & 15, tk = row >> 2, part = min(row & 3, 2);
-            if (r == 0 || (tk >> 1) == 1) {
+            if (!stay && (r == 0 || (tk >> 1) == 1)) {
                 const uint8_t *src = lds + (((tk & 1) * 8) * 4 + (lane >> 4)) * 48 + 16 * part;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) f[j] = *reinterpret_cast<const v4u *>(src + j * 4 * 48);
+                for (int j = 0; j < 8; ++j) f[j] = *reinterpret_cast<const v4u *>(src + j * MX_GRP);
             }
             if constexpr (DEN)
                 if (r == 0 || (lane >> 5) == 1) xexp = exps[(lane >> 4) & 1];
@@ -559,8 +572,9 @@ __device__ __forceinline__ f4v mx_mma16(uint32_t a0, uint32_t a1, uint32_t b0, u
 __device__ __forceinline__ float mx_sum3(const f4v &d) { return d[0] + (d[1] + d[2]); }
 
 // one unit's products (lane (r, c): weight row r, token c of each token tile); the groups' sums in two chains
-template <uint32_t TY, int NTILE>
-__device__ __forceinline__ void mx_unit(uint32_t *w, const v4u (&f)[NTILE][8], const float *sums,
+// fx(i, j): the operand of token tile i, group j
+template <uint32_t TY, int NTILE, class FX>
+__device__ __forceinline__ void mx_unit(uint32_t *w, const FX &fx, const float *sums,
                                         const typename MxX<TY>::Exp (&xexp)[NTILE], int lane, const uint8_t *tab, float *out) {
     using F = MX<TY>;
     const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -585,14 +599,15 @@ __device__ __forceinline__ void mx_unit(uint32_t *w, const v4u (&f)[NTILE][8], c
 #pragma unroll
         for (int i = 0; i < NTILE; ++i) {
             float &a = acc[i][j & 1], &n = mins[i][j & 1];
+            const v4u f = fx(i, j);
             if constexpr (F::SUB) {
-                const f4v d0 = mx_mma16(f[i][j].x, f[i][j].y, b.x, b.y), d1 = mx_mma16(f[i][j].z, f[i][j].w, b.z, b.w);
+                const f4v d0 = mx_mma16(f.x, f.y, b.x, b.y), d1 = mx_mma16(f.z, f.w, b.z, b.w);
                 a = __builtin_fmaf(s[0], mx_sum3(d0), a);
                 a = __builtin_fmaf(s[1], mx_sum3(d1), a);
                 n = __builtin_fmaf(m[0], xs[i][j >> 1][2 * j & 3], n);
                 n = __builtin_fmaf(m[1], xs[i][j >> 1][(2 * j + 1) & 3], n);
             } else {
-                const f4v d = mx_mma(f[i][j], b, zero);
+                const f4v d = mx_mma(f, b, zero);
                 if constexpr (F::CHAIN) {
                     // (a weight is a bf16 value: where it is infinite or NaN the product is hi's, while mid and lo,
                     // often zero, give NaN)
@@ -621,21 +636,22 @@ __device__ __forceinline__ void mx_unit(uint32_t *w, const v4u (&f)[NTILE][8], c
 
 // One weight's tiles blk, blk + nblk, ... for tokens t0 .. t0 + 4 NTILE - 1 (of nt).  W = waves of the workgroup, U =
 // units of a row; wave w sums units w UPW ..
-template <uint32_t TY, int NTILE, int UPW>
+template <uint32_t TY, int NTILE, int UPW, int MAXT>
 __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, const float *__restrict__ x, int cols, int t0, int nt,
                                         float *__restrict__ y, int blk, int nblk, uint8_t *lds) {
     using F = MX<TY>;
+    constexpr bool HALF = TY == QT_BF16, STAY = mx_stay<TY>(UPW, MAXT);
     const int tid = threadIdx.x, lane = tid & 63, W = blockDim.x >> 6;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint8_t *tab = lds;
-    constexpr int WAVE = mx_wave<TY>(UPW, NTILE), SUMS = mx_sums(F::MIN, F::SUB) / 4;  // (SUMS: floats)
+    constexpr int WAVE = mx_wave<TY>(UPW, NTILE, MAXT), SUMS = mx_sums(F::MIN, F::SUB) / 4;  // (SUMS: floats)
     uint8_t *mine = lds + mx_tab_bytes<TY>() + wv * WAVE;
-    float *sums = reinterpret_cast<float *>(mine + MX_X + 64);
+    int *exps = reinterpret_cast<int *>(mine + (STAY ? 2 : 1) * MX_X);
+    float *sums = reinterpret_cast<float *>(exps + 16);
     float *red = reinterpret_cast<float *>(lds + mx_tab_bytes<TY>() + W * WAVE);
     const int r16 = lane & 15, q = lane >> 4, ntiles = (rows + rt - 1) / rt;
     const int u0 = wv * UPW;
     const bool two = UPW == 1 || u0 + 1 < U;  // (UPW = 2) the last wave may have one unit only
-    constexpr bool HALF = TY == QT_BF16;
     const auto load = [&](int tile, int k, uint32_t *w, bool first = true, bool second = true) {
         const RP32 R = row_planes32(P, min(tile * rt + min(r16, rt - 1), rows - 1));
         if (first) F::load(R, min(u0 + k, U - 1), q, w);
@@ -643,7 +659,8 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
             if (second) F::load2(R, min(u0 + k, U - 1), q, w);
         __builtin_amdgcn_sched_barrier(0);  // (requested here, not where the words are first used)
     };
-    // x, then the first tile's words, then the table: everything is in flight before the first wait
+    // x, then the first tile's words, then the table are requested before the first wait (a second unit's words and half of
+    // a BF16 unit's after x is split: no registers before)
     MxX<TY> xr[UPW][NTILE];
 #pragma unroll
     for (int k = 0; k < UPW; ++k)
@@ -659,7 +676,7 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
     const auto tile = [&](int i) { return blk + i * nblk; };
     load(blk, 0, wa, true, false);
     mx_tab_fill<TY>(tab, tid, blockDim.x);
-    v4u f[UPW][NTILE][8];
+    v4u f[STAY ? 1 : UPW][NTILE][8];
     typename MxX<TY>::Exp xexp[UPW][NTILE];
     const bool one = mx_one<TY>(NTILE) && nt - t0 == 1;
     const auto rounds = [&](int i) { return nt - t0 - 4 * i > 2 ? 2 : 1; };
@@ -669,16 +686,23 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
         for (int i = 0; i < NTILE; ++i) {
             float *s = sums + (k * NTILE + i) * SUMS;
             xr[k][i].test(rounds(i), one);
-            if (one) xr[k][i].split1(lane, mine, f[k][i], xexp[k][i]);
-            else xr[k][i].split(rounds(i), lane, mine, f[k][i], s, xexp[k][i]);
+            const bool stay = STAY && k > 0;
+            v4u *to = f[stay ? 0 : k][i];
+            if (one) xr[k][i].split1(lane, mine, to, xexp[k][i]);
+            else xr[k][i].split(stay, rounds(i), lane, mine, to, exps, s, xexp[k][i]);
         }
     if constexpr (HALF) load(blk, 0, wa, false, true);
     if constexpr (UPW == 2) load(blk, 1, wb);
+    const uint8_t *f1 = mine + MxX<TY>::piece(rounds(0), lane);  // STAY (UPW = 2, NTILE = 1)
     if constexpr (mx_tab_bytes<TY>() > 0) lds_barrier();
     int it = 0;
     float acc[NTILE];
     const auto products = [&](int k, uint32_t *w) {
-        mx_unit<TY, NTILE>(w, f[k], sums + k * NTILE * SUMS, xexp[k], lane, tab, acc);
+        float *s = sums + k * NTILE * SUMS;
+        if (STAY && k > 0)
+            mx_unit<TY, NTILE>(w, [&](int, int j) { return *reinterpret_cast<const v4u *>(f1 + j * MX_GRP); }, s, xexp[k], lane, tab, acc);
+        else
+            mx_unit<TY, NTILE>(w, [&](int i, int j) { return f[STAY ? 0 : k][i][j]; }, s, xexp[k], lane, tab, acc);
         __builtin_amdgcn_sched_barrier(0);
     };
     const auto clear = [&]() {
@@ -753,22 +777,22 @@ template <uint32_t TY, int NTILE, int UPW, int MAXT>
 __global__ void __launch_bounds__(MAXT, mx_waves(NTILE, UPW, MAXT)) k_gemv_mx(PP P, int rows, int rt, int U, const float *__restrict__ x, int cols, int nt,
                                                   float *__restrict__ y) {
     extern __shared__ float4 xs[];
-    mx_walk<TY, NTILE, UPW>(P, rows, rt, U, x, cols, 4 * NTILE * blockIdx.y, nt, y, blockIdx.x, gridDim.x,
+    mx_walk<TY, NTILE, UPW, MAXT>(P, rows, rt, U, x, cols, 4 * NTILE * blockIdx.y, nt, y, blockIdx.x, gridDim.x,
                             reinterpret_cast<uint8_t *>(xs));
 }
 
-template <int NTILE, int I, int N, uint32_t TY, uint32_t... R>
+template <int NTILE, int MAXT, int I, int N, uint32_t TY, uint32_t... R>
 __device__ __forceinline__ void mx_grp_walk(const GParts<N> &ps, int blk, int U, const float *__restrict__ x, int cols,
                                             int nt, uint8_t *lds) {
-    if (blk < ps.p[I].nwg) mx_walk<TY, NTILE, 1>(ps.p[I].P, ps.p[I].rows, ps.p[I].rt, U, x, cols, 0, nt, ps.p[I].out, blk, ps.p[I].nwg, lds);
-    else if constexpr (sizeof...(R) > 0) mx_grp_walk<NTILE, I + 1, N, R...>(ps, blk - ps.p[I].nwg, U, x, cols, nt, lds);
+    if (blk < ps.p[I].nwg) mx_walk<TY, NTILE, 1, MAXT>(ps.p[I].P, ps.p[I].rows, ps.p[I].rt, U, x, cols, 0, nt, ps.p[I].out, blk, ps.p[I].nwg, lds);
+    else if constexpr (sizeof...(R) > 0) mx_grp_walk<NTILE, MAXT, I + 1, N, R...>(ps, blk - ps.p[I].nwg, U, x, cols, nt, lds);
 }
 // several weights over one x: workgroups [0, nwg_0) walk part 0, the next nwg_1 part 1, and so on
 template <int NTILE, int MAXT, uint32_t... TS>
 __global__ void __launch_bounds__(MAXT, mx_waves(NTILE, 1, MAXT)) k_gemv_mx_grp(GParts<sizeof...(TS)> ps, int U, const float *__restrict__ x, int cols,
                                                       int nt) {
     extern __shared__ float4 xs[];
-    mx_grp_walk<NTILE, 0, sizeof...(TS), TS...>(ps, blockIdx.x, U, x, cols, nt, reinterpret_cast<uint8_t *>(xs));
+    mx_grp_walk<NTILE, MAXT, 0, sizeof...(TS), TS...>(ps, blockIdx.x, U, x, cols, nt, reinterpret_cast<uint8_t *>(xs));
 }
 
 // workgroups of W waves and lds bytes that a CU holds (queried once per kernel and W)
@@ -795,7 +819,7 @@ inline int mx_tile_rows(int rows) {
 template <uint32_t TY, int NTILE, int UPW, int MAXT>
 int mx_launch(const QLayout &L, const uint8_t *packed, const float *x, int nt, float *y, hipStream_t st) {
     static int cache[17] = {};
-    const int U = L.cols / 256, W = (U + UPW - 1) / UPW, lds = mx_lds<TY>(W, UPW, NTILE), rt = mx_tile_rows(L.rows);
+    const int U = L.cols / 256, W = (U + UPW - 1) / UPW, lds = mx_lds<TY>(W, UPW, NTILE, MAXT), rt = mx_tile_rows(L.rows);
     const int halves = (nt + 4 * NTILE - 1) / (4 * NTILE), ntiles = (L.rows + rt - 1) / rt;
     int per_cu = 0;
     if (mx_per_cu(k_gemv_mx<TY, NTILE, UPW, MAXT>, cache, W, lds, per_cu)) return -1;
@@ -823,7 +847,7 @@ template <int NTILE, int MAXT, uint32_t... TS>
 int mx_grp_launch(const QLayout *const *L, const PP *P, float *const *y, const float *x, int nt, hipStream_t st) {
     constexpr int N = sizeof...(TS);
     static int cache[17] = {};
-    const int U = L[0]->cols / 256, W = U, lds = std::max({mx_lds<TS>(W, 1, NTILE)...});
+    const int U = L[0]->cols / 256, W = U, lds = std::max({mx_lds<TS>(W, 1, NTILE, MAXT)...});
     int per_cu = 0;
     if (mx_per_cu(k_gemv_mx_grp<NTILE, MAXT, TS...>, cache, W, lds, per_cu)) return -1;
     // Tiles are of one size for all parts.  `walk`, the most tiles that a workgroup takes, is the fewest for which the

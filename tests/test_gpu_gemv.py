@@ -480,3 +480,24 @@ def test_gemv_matrix_cores_waves_per_cu(fnlib):
     assert 1 < cus <= 416 and grid[4] == cus and grid[30] == 3 * cus and grid[0] >= cus, grid
     for wpc in (4, 10, 30):
         assert np.array_equal(y[wpc], y[0]), wpc
+
+
+@pytest.mark.parametrize("name", ["Q5_K", "Q6_K"])
+@pytest.mark.parametrize("cols", [6400, 8192])
+def test_gemv_matrix_cores_wide_rows_not_slower(fnlib, name, cols):
+    """Rows of 25 to 32 units, several tiles a workgroup: the matrix cores are not the slower path.  Bound: at 2 and 4
+    tokens they take 0.65 to 1.06 of the vector kernels' time (the deep walk, their plan for it); with registers spilled
+    to scratch they took 1.3 to 1.5 of it at 2."""
+    t, rows = TYPES[name], 20000
+    for nt in (2, 4):
+        def us():
+            return min(fnlib.bench_gemv(t, rows, cols, nt=nt, iters=20) for _ in range(3)) * 1e3
+
+        mx = us()
+        fnlib.gemv_override(kernel=3)
+        try:
+            vec = us()
+        finally:
+            fnlib.gemv_override(0)
+        _say(f"gemv wide rows {name} {rows}x{cols} nt={nt}: {mx:.1f} us, vector kernels {vec:.1f} us")
+        assert mx <= 1.2 * vec
