@@ -34,7 +34,7 @@
 //   Q6_K   20000 x 8192    30.5 / 33.6   51.1 / 36.4  130.5 /  58.1
 //   Q6_K     300 x 8192     6.5 /  7.4    9.8 /  9.5   19.3 /   9.6
 //   grouped: DeltaNet's qkv, z (Q6_K), alpha and beta  12.4 / 11.4   23.0 / 12.6   32.8 / 16.3
-//            attention's q, k, v and indexer           12.0 / 10.6   19.4 / 11.3   27.4 / 14.8
+//            attention's q, k, v and indexer           12.8 /  9.9   19.9 / 11.0   28.1 /  12.3
 //            the FFN's router, shared gate and up       5.2 /  5.4    6.7 /  6.4    9.2 /   7.5
 // Error against 64 bits over 1024 to 6144 columns: 0.6 to 1.1e-7 (the vector kernels 0.8 to 1.1e-7), Q6_K 2.0e-7 (2.1e-7).
 #pragma once
@@ -854,15 +854,24 @@ int mx_grp_launch(const QLayout *const *L, const PP *P, float *const *y, const f
     // workgroups are resident at once.  Where a CU holds two, the ones left over are shared out by tiles: the walk alone
     // would leave some CUs two workgroups and others one (DeltaNet set, one token: 16.6 us so, 11.7 shared out); where it
     // holds one, more of them only split x more often (8 tokens: 16.0 us by the walk, 18.3 shared out).
+    // `walk` is of the part with the lightest rows; the others walk fewer tiles, by their bytes: a CU streams a BF16 tile
+    // (128 KB at 4096 columns) in the time of three or four of IQ4_XS, and one workgroup with four of them was what the
+    // launch waited for (attention set, one token, in equal tiles / by bytes: 2560 columns 11.9 / 9.9 us, 4096 columns
+    // 19.3 / 12.2, where the vector kernels take 15.4; 8 tokens 15.9 / 12.3 and 21.2 / 15.2).
     const int budget = device_cus() * per_cu;
     GParts<N> ps;
     int tiles[N], w[N], all = 0, rows = 0, walk = 0, nwg = 0;
+    size_t light = L[0]->row_bytes;
+    for (int i = 1; i < N; ++i) light = std::min(light, L[i]->row_bytes);
     for (int i = 0; i < N; ++i) rows += L[i]->rows;
     const int rt = mx_tile_rows(rows);
     for (int i = 0; i < N; ++i) all += tiles[i] = (L[i]->rows + rt - 1) / rt;
     do {
         ++walk, nwg = 0;
-        for (int i = 0; i < N; ++i) nwg += w[i] = (tiles[i] + walk - 1) / walk;
+        for (int i = 0; i < N; ++i) {
+            const int k = std::max(1, (int) (walk * light / L[i]->row_bytes));
+            nwg += w[i] = (tiles[i] + k - 1) / k;
+        }
     } while (nwg > budget && nwg > N);
     // (a part of a few tiles, such as the 96 rows of alpha and beta, has a workgroup for each)
     nwg = 0;

@@ -501,3 +501,47 @@ def test_gemv_matrix_cores_wide_rows_not_slower(fnlib, name, cols):
             fnlib.gemv_override(0)
         _say(f"gemv wide rows {name} {rows}x{cols} nt={nt}: {mx:.1f} us, vector kernels {vec:.1f} us")
         assert mx <= 1.2 * vec
+
+
+def _group_us(fnlib, types, rows, cols, nt, iters=24):
+    """us of a grouped launch, weights cold (every call of the replayed graph reads its own copy)"""
+    packs = [[hiprt.Buf(fnlib.gemv_packed_bytes(t, r, cols), np.uint8) for t, r in zip(types, rows)] for _ in range(12)]
+    for k, c in enumerate(packs):
+        for p in c:
+            fnlib.fill_normal_dev(p.ptr, p.nbytes // 4, 40 + k)
+    x, ys = hiprt.Buf.empty((nt, cols)), [hiprt.Buf.empty((nt, r)) for r in rows]
+    fnlib.fill_normal_dev(x.ptr, nt * cols, 39)
+    hiprt.sync()
+    st = hiprt.Stream()
+
+    def calls():
+        for k in range(iters):
+            fnlib.gemv_group_dev(types, rows, cols, [p.ptr for p in packs[k % 12]], x.ptr, nt, [y.ptr for y in ys], st.handle)
+
+    g, best = hiprt.Graph(st, calls), 1e9
+    for _ in range(4):
+        e0, e1 = hiprt.Event(), hiprt.Event()
+        e0.record(st)
+        g.launch()
+        e1.record(st)
+        e1.sync()
+        best = min(best, e1.ms_since(e0) / iters * 1e3)
+    g.destroy()
+    st.destroy()
+    return best
+
+
+def test_gemv_group_matrix_cores_not_slower(fnlib):
+    """The attention set at 4096 columns, one token, with its BF16 part of four times the bytes a row: the grouped launch
+    on the matrix cores is not the slower path.  Bound: 0.8 of the vector kernels' time; 1.25 with a workgroup's share
+    counted in tiles alone."""
+    types, rows = [TYPES["IQ4_XS"], TYPES["IQ4_XS"], TYPES["Q6_K"], TYPES["BF16"]], [12288, 512, 512, 640]
+    _say("gemv group, matrix cores and vector kernels, attention set at 4096 columns")
+    mx = _group_us(fnlib, types, rows, 4096, 1)
+    fnlib.gemv_override(kernel=4)
+    try:
+        vec = _group_us(fnlib, types, rows, 4096, 1)
+    finally:
+        fnlib.gemv_override(0)
+    _say(f"  {mx:.1f} us, vector kernels {vec:.1f} us")
+    assert mx <= 1.1 * vec
