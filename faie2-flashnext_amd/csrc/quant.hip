@@ -175,13 +175,21 @@ bool gemv_planes_fit(const QLayout &L) {
 
 // Rows of 4 to 32 whole units of 256 values: below, a workgroup would be fewer than 4 waves for a tile; above, the waves
 // (at most 16) would hold more than two units of x, for which the registers do not reach.  A BF16 unit takes 128 bytes
-// of a lane, so two of them do not fit beside x either.  The other formats (the routed experts') have no decode there.
+// of a lane, so two of them do not fit beside x either.  IQ3_S stops at 25 units: its decode, two codebook lookups and a
+// sign mask for 8 values, costs more than its loads where all of a CU's 14 to 16 waves do it at once (vector kernels /
+// matrix cores, us at 1, 2 and 8 tokens: 20000 x 6400 24.9 / 25.5, 28.0 / 25.8, 107 / 45; x 6656 25.4 / 28.4, 30.9 / 28.9,
+// 112 / 51; x 8192 28.1 / 38.0, 33.5 / 39.8, 116 / 69; 300 x 8192 6.7 / 8.5, 8.0 / 9.2, 18.4 / 10.6).  The other formats
+// (the routed experts') have no decode there.
+// The line may not depend on the tokens (every token has the bits of a one-token call), and in places one token is the
+// dearer for what several gain: short weights of 17 units and more (300 x 8192, 1 / 4 / 8 tokens: Q8_0 5.7 / 6.3, 9.2 /
+// 8.3, 17.8 / 8.5; Q6_K 6.5 / 7.4, 9.8 / 9.5, 19.3 / 9.6), 600 x 4096 in the K-quants and IQ3_S (Q6_K 4.9 / 5.4, 6.6 /
+// 6.5, 9.5 / 9.1) and Q6_K 20000 x 8192 (30.5 / 33.6, 51 / 36, 130 / 58).
 bool gemv_mx_use(const QLayout &L) {
     if (g_ov_lpr || g_ov_kernel || L.cols % 256 || L.cols < 4 * 256 || L.cols > 32 * 256) return false;
     switch (L.type) {
         case QT_BF16: return L.cols <= 16 * 256;
-        case QT_Q8_0: case QT_IQ4_NL: case QT_IQ4_XS: case QT_Q4_K: case QT_Q5_K: case QT_Q6_K:
-        case QT_IQ3_S: return true;
+        case QT_IQ3_S: return L.cols <= 25 * 256;
+        case QT_Q8_0: case QT_IQ4_NL: case QT_IQ4_XS: case QT_Q4_K: case QT_Q5_K: case QT_Q6_K: return true;
         default: return false;
     }
 }

@@ -545,3 +545,22 @@ def test_gemv_group_matrix_cores_not_slower(fnlib):
         fnlib.gemv_override(0)
     _say(f"  {mx:.1f} us, vector kernels {vec:.1f} us")
     assert mx <= 1.1 * vec
+
+
+@pytest.mark.parametrize("cols,matrix", [(6144, True), (6400, True), (6656, False), (8192, False)])
+def test_gemv_iq3s_path_by_columns(fnlib, cols, matrix):
+    """IQ3_S rows of up to 25 units run on the matrix cores, wider ones keep the vector kernels (the faster path for one
+    token there) and their bits, whatever the tokens."""
+    t, rows = TYPES["IQ3_S"], 77
+    _say(f"gemv IQ3_S {rows}x{cols}: matrix cores {matrix}")
+    raw = random_finite(t, rows, cols, np.random.default_rng(17))
+    x = np.random.default_rng(18).standard_normal((8, cols)).astype(np.float32)
+    auto = [fnlib.gemv(t, raw, rows, cols, x[:nt]) for nt in (1, 8)]
+    fnlib.gemv_override(kernel=4)
+    try:
+        vec = fnlib.gemv(t, raw, rows, cols, x)
+    finally:
+        fnlib.gemv_override(0)
+    for y in auto:
+        assert np.array_equal(y, vec[:len(y)]) == (not matrix)
+        assert oracle.relerr(y, oracle.gemv(t, raw, rows, cols, x[:len(y)])) <= TOL
