@@ -320,3 +320,20 @@ def test_attn_multi_token_query_out_of_range(fnlib, nq, nt):
         og = fnlib.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc.copy(), case.Vc.copy(), case.pos)
         ref, _, _ = oracle.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc, case.Vc, case.pos)
         assert oracle.relerr(og, ref) <= 2e-6
+
+
+@pytest.mark.parametrize("nq,nt", [(16, 16), (24, 10)])
+def test_attn_multi_token_growing_scores_fp32_walk(fnlib, nq, nt):
+    """test_attn_multi_token_growing_scores on 97 to 128 query rows, which walk in fp32 on four row groups of two row
+    blocks.  Bound: the keys that count have the largest scores, three times the spread of q.k (|q| |k| / 16 = 16 * 336 /
+    16), so 1000; a score is 64 sums of 4 products, rounded at 2^-24 of that, and then divided by 16: 8 * 2^-24 * 1000 /
+    16 = 3e-5 in a probability where the roundings add as a root (the smaller calls' 1e-5 is what they show)."""
+    _say(f"attn multi-token growing scores, fp32 walk nq={nq} nt={nt}")
+    L = 2000
+    case = _mt_case(2, nq, 2, nt, [L - nt, 1234], 2048, seed=91 + nq + nt)
+    ramp = (1.0 + 20.0 * np.arange(2048) / L).astype(np.float32)
+    case.Kc *= ramp[None, :, None, None]
+    case.Kc[0, 1500] *= 40.0
+    og = fnlib.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc.copy(), case.Vc.copy(), case.pos)
+    ref, _, _ = oracle.attn(case.qg, case.k, case.v, case.wq, case.wk, case.Kc, case.Vc, case.pos)
+    assert oracle.relerr(og, ref) <= 3e-5

@@ -564,3 +564,73 @@ def test_gemv_iq3s_path_by_columns(fnlib, cols, matrix):
     for y in auto:
         assert np.array_equal(y, vec[:len(y)]) == (not matrix)
         assert oracle.relerr(y, oracle.gemv(t, raw, rows, cols, x[:len(y)])) <= TOL
+
+
+@pytest.mark.parametrize("name", MX_TYPES)
+@pytest.mark.parametrize("rows,cols", [(40, 2560), (20, 4608)])
+def test_gemv_matrix_cores_specials_all_formats(fnlib, name, rows, cols):
+    """test_gemv_matrix_cores_specials over every format of the matrix cores and rows of two units a wave: infinities and
+    NaNs in x come out where the vector kernels put them (through the K-quants' scale of x and their minimum term too),
+    a token beside them is untouched."""
+    if name == "BF16" and cols > 4096:
+        cols = 4096
+    t = TYPES[name]
+    rng = np.random.default_rng(19)
+    _say(f"gemv matrix cores, infinities and NaNs, {name} {rows}x{cols}")
+    raw = random_finite(t, rows, cols, rng)
+    if name == "BF16":
+        raw = (rng.standard_normal(rows * cols).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).view(np.uint8)
+    x = rng.standard_normal((6, cols)).astype(np.float32)
+    clean = fnlib.gemv(t, raw, rows, cols, x)
+    x[1, 100], x[2, 200], x[3, 300], x[5, cols - 1] = np.inf, -np.inf, np.nan, np.inf
+    y = fnlib.gemv(t, raw, rows, cols, x)
+    fnlib.gemv_override(kernel=4)
+    try:
+        yv = fnlib.gemv(t, raw, rows, cols, x)
+    finally:
+        fnlib.gemv_override(0)
+    for i in (0, 4):
+        assert np.array_equal(y[i].view(np.uint32), clean[i].view(np.uint32))
+    assert np.array_equal(np.isnan(y), np.isnan(yv))
+    inf = np.isinf(yv)
+    assert np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], yv[inf])
+
+
+@pytest.mark.parametrize("parts", [[("IQ4_XS", 1040), ("IQ3_S", 520), ("BF16", 77)], [("BF16", 96), ("Q6_K", 3000), ("IQ4_XS", 5000)],
+                                   [("Q6_K", 512), ("IQ4_XS", 9000), ("IQ4_XS", 17), ("BF16", 640)]])
+@pytest.mark.parametrize("cols", [1024, 2560, 3328, 4096])
+@pytest.mark.parametrize("nt", [1, 5, 8])
+def test_gemv_group_matrix_cores_own_bits(fnlib, parts, cols, nt):
+    """On the matrix cores (1024 to 4096 columns) every part of a grouped launch has its own GEMV's bits, whatever tile
+    height the group and the weight alone take."""
+    types, rows = [TYPES[n] for n, _ in parts], [r for _, r in parts]
+    _say(f"gemv group on the matrix cores {parts} cols={cols} nt={nt}")
+    rng = np.random.default_rng(20)
+    raws = [random_finite(t, r, cols, rng) for t, r in zip(types, rows)]
+    x = rng.standard_normal((nt, cols)).astype(np.float32)
+    for t, r, raw, y in zip(types, rows, raws, _group_run(fnlib, types, rows, raws, cols, x)):
+        assert np.array_equal(y.view(np.uint32), fnlib.gemv(t, raw, r, cols, x).view(np.uint32)), (t, r)
+
+
+@pytest.mark.parametrize("parts", [[("IQ4_XS", 4000), ("IQ3_S", 2100), ("BF16", 77)], [("BF16", 96), ("Q6_K", 2100), ("IQ4_XS", 4000)],
+                                   [("Q6_K", 512), ("IQ4_XS", 7000), ("IQ4_XS", 17), ("BF16", 640)]])
+@pytest.mark.parametrize("cols,forced", [(512, False), (768, False), (4352, False), (2560, True), (4096, True)])
+@pytest.mark.parametrize("nt", [1, 3, 8])
+def test_gemv_group_vector_kernels(fnlib, parts, cols, forced, nt):
+    """The grouped vector kernels, which the sets keep below 1024 columns, above 4096 while x fits the LDS, and under a
+    forced plan: every set, several row-sets a wave, against float64 math, and a token's bits in every call."""
+    types, rows = [TYPES[n] for n, _ in parts], [r for _, r in parts]
+    _say(f"gemv group on the vector kernels {parts} cols={cols} nt={nt} forced={forced}")
+    rng = np.random.default_rng(22)
+    raws = [random_finite(t, r, cols, rng) for t, r in zip(types, rows)]
+    x = rng.standard_normal((nt, cols)).astype(np.float32)
+    if forced:
+        fnlib.gemv_override(kernel=4)
+    try:
+        ys = _group_run(fnlib, types, rows, raws, cols, x)
+        last = _group_run(fnlib, types, rows, raws, cols, x[-1:])
+    finally:
+        fnlib.gemv_override(0)
+    for t, r, raw, y, y1 in zip(types, rows, raws, ys, last):
+        assert oracle.relerr(y, oracle.gemv(t, raw, r, cols, x)) <= TOL, (t, r)
+        assert np.array_equal(y[-1].view(np.uint32), y1[0].view(np.uint32)), (t, r)
