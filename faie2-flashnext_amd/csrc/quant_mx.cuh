@@ -41,8 +41,6 @@
 
 #include "quant_impl.cuh"
 
-#include <type_traits>
-
 namespace fn {
 namespace {
 
@@ -423,17 +421,16 @@ template <uint32_t TY> constexpr bool mx_one(int ntile) { return ntile == 1 && !
 // it, split() makes the wave's A operands of it.  f[j] is lane (m, q)'s operand of group j: row m = token m / 4, part
 // m % 4 (the unused fourth row reads lo again).  Two tokens a round through the wave's LDS, 8 values a lane.
 //   sums (MIN), in the LDS: [token][group] of x (SUB: [token][group][half]);
-//   xexp: the scale of x, a power of two, by unit and token.  DEN: x is scaled by 2^xexp, of the unit's largest.  Else
-//   xexp is the mask of the result's lanes (16 a token) whose unit is scaled by 2^UP, because all of it is below 2^-63, so
-//   that values too small for an exact split (split3) have one.  A unit with a larger value is not scaled: what it may
-//   lose is below 2^-133, 2^-70 of that value.  No sum overflows by it: scaled values are below 2^-10, less than 1 / 256
-//   (the values of a unit) beside any weight.  On an x of size 1e-36: 5e-5 off 64 bits unscaled, 1e-7 scaled.  The test
-//   costs up to 0.2 us at 8 tokens (IQ4_XS 640 x 2560 6.45 / 6.66 us; one token 4.19 either way), the scaling nothing.
+//   The scale of x, a power of two.  DEN: x is scaled by 2^xexp, of the unit's largest.  Else a token's slice of x (the
+//   wave's one or two units) is scaled by 2^MX_UP where all of it is below 2^-63 (up: the lanes of such tokens, by round),
+//   so that values too small for an exact split (split3) have one.  A slice with a larger value is not scaled: what it may
+//   lose is below 2^-133, 2^-70 of that value.  No sum overflows by it: scaled values are below 2^-10, less than 1 / 512
+//   (the values of two units) beside any weight.  On an x of size 1e-36: 5e-5 off 64 bits unscaled, 1e-7 scaled.
 //   Scaled under a branch instead, or split a second time where bits are lost, it cost 30 registers.
+constexpr int MX_UP = 53;
 template <uint32_t TY> struct MxX {
     static constexpr int MAP = MX<TY>::MAP, NS = MX<TY>::SUB ? 2 : 1;
     static constexpr bool MIN = MX<TY>::MIN, DEN = MX<TY>::DEN;
-    using Exp = std::conditional_t<DEN, int, uint64_t>;
     f4v a[2], b[2];
     __device__ __forceinline__ void load(const float *__restrict__ x, int cols, int u, int t0, int nt, int lane, bool single) {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
@@ -465,26 +462,8 @@ template <uint32_t TY> struct MxX {
     }
     // x's scale: the largest magnitude (of the token's 256 values) to just under 2^120
     static __device__ __forceinline__ int scale_of(float mx) { return 246 - (int) (__float_as_uint(mx) >> 23); }
-    static constexpr int UP = 53;
-    // test(): the lanes whose token's unit is scaled, by round.  A unit is not if a value is at least 2^-63 (its exponent's
-    // first or second bit is set), an infinity or a NaN.
-    uint64_t up[2];
-    __device__ __forceinline__ void test(int rounds, bool one) {
-        if constexpr (DEN) return;
-        const auto large = [](const f4v &c) {
-            return __float_as_uint(c[0]) | __float_as_uint(c[1]) | __float_as_uint(c[2]) | __float_as_uint(c[3]);
-        };
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            if (r >= rounds) break;
-            const uint64_t big = __ballot(((one ? large(a[0]) : large(a[r]) | large(b[r])) & 0x60000000u) != 0);
-            const uint32_t t0 = (uint32_t) big, t1 = (uint32_t) (big >> 32);
-            const uint32_t u0 = (one ? t0 | t1 : t0) ? 0u : ~0u, u1 = (one ? t0 | t1 : t1) ? 0u : ~0u;
-            up[r] = (uint64_t) u1 << 32 | u0;
-        }
-    }
-    template <int N> __device__ __forceinline__ void scale_up(int r, float *v) const {
-        const float sc = __builtin_amdgcn_inverse_ballot_w64(up[r]) ? __builtin_ldexpf(1.0f, UP) : 1.0f;
+    template <int N> static __device__ __forceinline__ void scale_up(uint64_t up, float *v) {
+        const float sc = __builtin_amdgcn_inverse_ballot_w64(up) ? __builtin_ldexpf(1.0f, MX_UP) : 1.0f;
 #pragma unroll
         for (int k = 0; k < N; ++k) v[k] *= sc;
     }
@@ -500,12 +479,11 @@ template <uint32_t TY> struct MxX {
         return (rounds > 1 ? (tk >> 1) * MX_X : 0) + ((tk & 1) * 32 + (lane >> 4)) * 48 + 16 * part;
     }
     // split() of one token, the same bits with half the work a lane (mx_one)
-    __device__ __forceinline__ void split1(int lane, uint8_t *lds, v4u *f, Exp &xexp) const {
+    __device__ __forceinline__ void split1(int lane, uint8_t *lds, v4u *f, const uint64_t *up) const {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
         float v[4] = {a[0][0], a[0][1], a[0][2], a[0][3]};
         uint32_t h[2], m[2], l[2];
-        xexp = up[0];
-        scale_up<4>(0, v);
+        scale_up<4>(up[0], v);
         split_n<4>(v, h, m, l);
         v2u *dst = reinterpret_cast<v2u *>(lds + (gl * 4 + q) * 48 + 8 * ts);
         dst[0] = v2u{h[0], h[1]};
@@ -517,9 +495,9 @@ template <uint32_t TY> struct MxX {
         for (int j = 0; j < 8; ++j) f[j] = *reinterpret_cast<const v4u *>(src + j * MX_GRP);
         fence();
     }
-    __device__ __forceinline__ void split(bool stay, int rounds, int lane, uint8_t *lds, v4u *f, int *exps, float *sums, Exp &xexp) const {
+    __device__ __forceinline__ void split(bool stay, int rounds, int lane, uint8_t *lds, v4u *f, int *exps, float *sums, const uint64_t *up,
+                                          int &xexp) const {
         const int q = lane & 3, gl = (lane >> 2) & 7, ts = lane >> 5;
-        if constexpr (!DEN) xexp = 0;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             if (r >= rounds) break;
@@ -550,8 +528,7 @@ template <uint32_t TY> struct MxX {
                 for (int k = 0; k < 8; ++k) v[k] = ldexpf(v[k], e);
                 if ((lane & 31) == 0) exps[ts] = e;
             } else {
-                scale_up<8>(r, v);
-                xexp |= ((up[r] & 0xFFFFull) | ((up[r] >> 32) & 0xFFFFull) << 16) << (32 * r);
+                scale_up<8>(up[r], v);
             }
             uint32_t h[4], m[4], l[4];
             split_n<8>(v, h, m, l);
@@ -585,7 +562,7 @@ __device__ __forceinline__ float mx_sum3(const f4v &d) { return d[0] + (d[1] + d
 // fx(i, j): the operand of token tile i, group j
 template <uint32_t TY, int NTILE, class FX>
 __device__ __forceinline__ void mx_unit(uint32_t *w, const FX &fx, const float *sums,
-                                        const typename MxX<TY>::Exp (&xexp)[NTILE], int lane, const uint8_t *tab, float *out) {
+                                        const int (&xexp)[NTILE], int lane, const uint8_t *tab, float *out) {
     using F = MX<TY>;
     const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
     float acc[NTILE][2], mins[NTILE][2];
@@ -637,8 +614,6 @@ __device__ __forceinline__ void mx_unit(uint32_t *w, const FX &fx, const float *
             F::super(w, d, dm);
             // (the power of two last: before d, a sum near fp32's smallest values would lose bits that d v has)
             v = __builtin_fmaf(-dm, mins[i][0] + mins[i][1], ldexpf(d * v, 133 - F::SHIFT - xexp[i]));
-        } else {
-            v *= __builtin_amdgcn_inverse_ballot_w64(xexp[i]) ? __builtin_ldexpf(1.0f, -MxX<TY>::UP) : 1.0f;
         }
         out[i] += v;
     }
@@ -692,19 +667,54 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
     if constexpr (UPW == 2) mx_tab_load<TY>(tid, blockDim.x, points);
     mx_tab_fill<TY>(tab, tid, blockDim.x, points);
     v4u f[STAY ? 1 : UPW][NTILE][8];
-    typename MxX<TY>::Exp xexp[UPW][NTILE];
+    int xexp[UPW][NTILE];
+    uint64_t up[NTILE][2] = {}, down[NTILE] = {};  // the lanes of scaled tokens: of x, by round, and of the results
     const bool one = mx_one<TY>(NTILE) && nt - t0 == 1;
     const auto rounds = [&](int i) { return nt - t0 - 4 * i > 2 ? 2 : 1; };
+    if constexpr (!F::DEN) {
+        // A value of at least 2^-63 has its exponent's first or second bit set (an infinity or a NaN too).  First one value a
+        // lane, of all tokens at once: a lane of each half with no smaller one settles it (all values of every unit and
+        // round, looked at before its split, cost 0.1 to 0.2 us at 8 tokens: BF16 96 x 2560 4.86 unscaled / 5.07 / 4.80 so).
+        const auto large = [&](int i, int r, bool all) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int k = 0; k < UPW; ++k) {
+                const f4v &a = xr[k][i].a[r], &b = xr[k][i].b[r];
+                m |= __float_as_uint(a[0]);
+                if (!all) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m |= __float_as_uint(a[e]) | (one ? 0u : __float_as_uint(b[e]));
+            }
+            return m & 0x60000000u;
+        };
+        uint32_t least = ~0u;
+#pragma unroll
+        for (int i = 0; i < NTILE; ++i) {
+            least = min(least, large(i, 0, false));
+            if (rounds(i) > 1) least = min(least, large(i, 1, false));
+        }
+        const uint64_t some = __ballot(least != 0);
+        if (one ? some == 0 : (uint32_t) some == 0 || (some >> 32) == 0)
+#pragma unroll
+            for (int i = 0; i < NTILE; ++i)
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    if (r >= rounds(i)) break;
+                    const uint64_t big = __ballot(large(i, r, true) != 0);
+                    const uint64_t b0 = one ? big : (uint32_t) big, b1 = one ? big : big >> 32;
+                    up[i][r] = (b0 ? 0 : 0xFFFFFFFFull) | (b1 ? 0 : 0xFFFFFFFFull << 32);
+                    down[i] |= ((up[i][r] & 0xFFFF) | ((up[i][r] >> 32) & 0xFFFF) << 16) << (32 * r);
+                }
+    }
 #pragma unroll
     for (int k = 0; k < UPW; ++k)
 #pragma unroll
         for (int i = 0; i < NTILE; ++i) {
             float *s = sums + (k * NTILE + i) * SUMS;
-            xr[k][i].test(rounds(i), one);
             const bool stay = STAY && k > 0;
             v4u *to = f[stay ? 0 : k][i];
-            if (one) xr[k][i].split1(lane, mine, to, xexp[k][i]);
-            else xr[k][i].split(stay, rounds(i), lane, mine, to, exps, s, xexp[k][i]);
+            if (one) xr[k][i].split1(lane, mine, to, up[i]);
+            else xr[k][i].split(stay, rounds(i), lane, mine, to, exps, s, up[i], xexp[k][i]);
         }
     if constexpr (HALF) load(blk, 0, wa, false, true);
     if constexpr (UPW == 2) load(blk, 1, wb);
@@ -727,7 +737,10 @@ __device__ __forceinline__ void mx_walk(const PP &P, int rows, int rt, int U, co
     const auto finish = [&](int tile) {
         float *buf = red + (it & 1) * (16 * NTILE * 64);
 #pragma unroll
-        for (int i = 0; i < NTILE; ++i) buf[(wv * NTILE + i) * 64 + lane] = acc[i];
+        for (int i = 0; i < NTILE; ++i) {
+            if constexpr (!F::DEN) acc[i] *= __builtin_amdgcn_inverse_ballot_w64(down[i]) ? __builtin_ldexpf(1.0f, -MX_UP) : 1.0f;
+            buf[(wv * NTILE + i) * 64 + lane] = acc[i];
+        }
         lds_barrier();  // (the buffers alternate: this one is written again only after the next tile's barrier)
         // one wave a token tile (in turn) sums the waves' words, a token at a time: lane (r, g) those of waves g, g + 4,
         // g + 8, g + 12 of row r (room for 16 is there; those past the last wave are read and left out), then the four
