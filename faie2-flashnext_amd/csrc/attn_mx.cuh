@@ -1,13 +1,17 @@
 // The walk of k_attn_split_mt on the bf16 matrix cores (included by attn.hip, after its fp32 walk).
 //
 // Every fp32 operand is the sum of three bf16 values (hi, mid, lo: 8 bits each, rounded to nearest, so the sum is
-// exact) and a product takes the six of the nine part products that reach fp32's precision: hi hi, hi mid, mid hi, hi
-// lo, lo hi, mid mid; what is left out is below 2^-26 of a product.  On v_mfma_f32_16x16x32_bf16 six of them take 96
-// cycles for 32 contraction slots where v_mfma_f32_16x16x4f32 takes 256.
+// exact, down to 2^-110: what lies below is looked after at MX_PUP) and a product takes the six of the nine part products
+// that reach fp32's precision: hi hi, hi mid, mid hi, hi lo, lo hi, mid mid.  What is left out, mid lo + lo mid + lo lo,
+// is at most 2^-24 of a product (mid reaches 2^-8 of an operand, lo 2^-17), half a unit of its last fp32 place, and about
+// 2^-28 in the mean; the sums' error against 64 bits is 8.4e-7 to 8.5e-7 where fp32 products gave 8.9e-7.  On
+// v_mfma_f32_16x16x32_bf16 six of them take 96 cycles for 32 contraction slots where v_mfma_f32_16x16x4f32 takes 256.
 // What bounds it: per 32 keys and 32 query rows a wave issues 384 products (6,144 cycles) and about as many cycles of
 // VALU for the split of K and V (11 instructions for two values), so the two are interleaved by hand: step s of the
 // walk issues 12 products on the operand split during step s - 1, and between them the 12 pieces of the split of step
-// s + 1's operand.  A step is 32 dims of a 16-key block's scores, or one 16-dim tile of P.V over 32 keys.
+// s + 1's operand.  A step is 32 dims of a 16-key block's scores, or one 16-dim tile of P.V over 32 keys.  By the
+// counters of an 8-token step over 16 x 32K the matrix cores are busy 41 % of the time, the vector units 52 %, both at
+// once 17 %.
 // Contraction slots (free to permute as long as both operands agree), lane l, 8 a lane: of the scores, chunks 4 (2u)
 // + l/16 and 4 (2u + 1) + l/16 of the row (the cache's 16-byte chunks); of P.V, keys 4(l/16) + 0..3 of the first and
 // of the second 16-key block, which the scores leave in the lane that needs them.
@@ -16,8 +20,8 @@
 // it split: K of the next 16 keys, V of the other 128 dims; loads are in flight for about 14 steps, in 128 registers
 // (with all 256 dims of V held, 192 registers, the walk spills).
 // Measured on MI355X, layer step, fp32 walk / this one in us (sequences, keys, tokens, query heads; 2 kv heads): 16, 32K,
-// 8, 16: 667 / 521; 16, 32K, 4, 16: 354 / 319; 4, 16K, 6, 24: 185 / 124; 1, 128K, 8, 24: 351 / 221; 1, 4K, 4, 16: 34.0 /
-// 29.9; 64, 2K, 3, 16: 119 / 108; 1, 130, 3, 16: 28.3 / 25.9.  Faster at every shape tried, so the rule asks for no more
+// 8, 16: 667 / 520; 16, 32K, 4, 16: 354 / 318; 4, 16K, 6, 24: 185 / 124; 1, 128K, 8, 24: 351 / 218; 1, 4K, 4, 16: 34.0 /
+// 29.3; 64, 2K, 3, 16: 119 / 107; 1, 130, 3, 16: 28.3 / 25.6.  Faster at every shape tried, so the rule asks for no more
 // than that Q fits.  Up to 16 rows half of the products would be padding and the K/V reads bound the fp32 walk: it stays.
 
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));

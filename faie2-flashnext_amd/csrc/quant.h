@@ -93,9 +93,10 @@ int gemv_split_launch(const QLayout &L, const uint8_t *packed, const float *x, i
 
 // Several weights with the same cols over one x (y_i[t][r] = W_i[r] . x[t]): one launch when their formats form one
 // of the sets built as a group (quant_grp.hip) and x of nt tokens fits the LDS, else one GEMV launch per weight.
-// A grouped launch sums every row with the group's lanes per row (the GEMV's arithmetic with that lpr), so a
-// weight's results may differ in the last bits from its own GEMV's; which path runs depends on the shapes and
-// formats only, never on nt.
+// On the matrix cores (1024 to 4096 columns) every weight gets its own GEMV's bits.  The vector kernels' grouped launch
+// sums every row with the group's lanes per row (the GEMV's arithmetic with that lpr), so a weight's results may
+// differ there in the last bits from its own GEMV's.  Which path runs depends on the shapes and formats only, never
+// on nt.
 struct GemvPart {
     const QLayout *L;
     const uint8_t *packed;

@@ -183,7 +183,7 @@ bool gemv_planes_fit(const QLayout &L) {
 // The line may not depend on the tokens (every token has the bits of a one-token call), and in places one token is the
 // dearer for what several gain: short weights of 17 units and more (300 x 8192, 1 / 4 / 8 tokens: Q8_0 5.7 / 6.3, 9.2 /
 // 8.3, 17.8 / 8.5; Q6_K 6.5 / 7.4, 9.8 / 9.5, 19.3 / 9.6), 600 x 4096 in the K-quants and IQ3_S (Q6_K 4.9 / 5.4, 6.6 /
-// 6.5, 9.5 / 9.1) and Q6_K 20000 x 8192 (30.5 / 33.6, 51 / 36, 130 / 58).
+// 6.5, 9.5 / 9.1), Q6_K 20000 x 8192 (30.5 / 33.6, 51 / 36, 130 / 58) and, by 2 %, Q8_0 2048 x 4096 and the FFN's group.
 bool gemv_mx_use(const QLayout &L) {
     if (g_ov_lpr || g_ov_kernel || L.cols % 256 || L.cols < 4 * 256 || L.cols > 32 * 256) return false;
     switch (L.type) {

@@ -22,20 +22,26 @@
 // gets the bits of a one-token call, and a weight of a grouped launch those of its own.
 //
 // What bounds it: at one token the launch, x's round trip and split and the weight's first round trip (about 4 us, the
-// whole of a small weight), then the decode, 2 to 3 vector instructions a value; the matrix cores are busy a quarter of
-// that.  Cold weights, us a call, the vector kernels / this, at 1, 4 and 8 tokens:
-//   IQ4_XS 10240 x 2560    10.1 /  8.7   17.1 /  9.5   24.5 /  11.3
-//   Q6_K    6144 x 2560     9.2 /  8.8   11.4 / 10.1   16.2 /  10.9
-//   Q8_0    2560 x 6144     8.9 /  8.7   13.5 / 10.0   20.3 /  13.8
-//   BF16      96 x 2560     4.6 /  4.2    6.0 /  4.8    8.6 /   5.8
-//   Q4_K   20000 x 8192    27.4 / 22.8   47.9 / 24.3  124.0 /  33.5
-//   Q5_K  248320 x 2560   104.8 / 98.9  183.4 / 105.0  291.3 / 139.6
-//   Q5_K    2560 x 8192     9.8 /  8.9   14.1 / 11.2   28.6 /  16.3
-//   Q6_K   20000 x 8192    30.5 / 33.6   51.1 / 36.4  130.5 /  58.1
-//   Q6_K     300 x 8192     6.5 /  7.4    9.8 /  9.5   19.3 /   9.6
-//   grouped: DeltaNet's qkv, z (Q6_K), alpha and beta  12.4 / 11.4   23.0 / 12.6   32.8 / 16.3
-//            attention's q, k, v and indexer           12.8 /  9.9   19.9 / 11.0   28.1 /  12.3
-//            the FFN's router, shared gate and up       5.2 /  5.4    6.7 /  6.4    9.2 /   7.5
+// whole of a small weight), then the decode.  By the counters of IQ4_XS 10240 x 2560 at 1 / 8 tokens: 4.1 / 5.5 vector
+// instructions a value, x's split included, the vector units busy 46 / 39 % of the time and the matrix cores 5 / 7 %.
+// One weight decode serves all tokens of a call up to 4096 columns; wider rows (two units a wave) take 4 tokens at a
+// time, so that a call of 5 to 8 reads and decodes the weight twice.
+// Cold weights, us a call, the vector kernels / this, at 1, 4 and 8 tokens:
+//   IQ4_XS 10240 x 2560     9.2 /  7.6   15.9 /  8.7   23.0 /  10.7
+//   Q6_K    6144 x 2560     8.4 /  7.7   10.7 /  9.0   15.3 /  10.2
+//   Q8_0    2560 x 6144     7.9 /  7.8   12.4 /  9.2   19.1 /  13.1
+//   Q8_0    2048 x 4096     5.8 /  6.0    7.4 /  7.0    9.8 /   8.6
+//   BF16      96 x 2560     4.4 /  4.0    5.8 /  4.8    8.3 /   5.9
+//   IQ3_S    640 x 2560     5.6 /  5.1    6.9 /  5.9    9.6 /   7.1
+//   Q4_K   20000 x 8192    25.4 / 21.6   46.0 / 23.6  122.6 /  37.6
+//   Q5_K  248320 x 2560   109.9 /102.8  176.8 / 107.1  271.2 / 130.8
+//   Q5_K    2560 x 8192     9.6 /  8.7   13.7 / 10.9   27.7 /  15.9
+//   Q6_K   20000 x 8192    30.0 / 35.2   51.5 / 35.6  130.1 /  53.8
+//   Q6_K     300 x 8192     6.5 /  7.3    9.8 /  9.4   19.3 /   9.6
+//   grouped: DeltaNet's qkv, z (Q6_K), alpha and beta  13.3 / 11.8   23.4 / 12.9   33.3 / 15.6
+//            attention's q, k, v and indexer           12.9 / 10.0   20.0 / 11.1   27.9 / 12.5
+//            the FFN's router, shared gate and up       6.2 /  6.3    7.6 /  6.9    9.9 /  7.5
+//            the same at 4096 columns                   6.8 /  7.6    8.4 /  8.3   10.7 /  9.4
 // Error against 64 bits over 1024 to 6144 columns: 0.6 to 1.1e-7 (the vector kernels 0.8 to 1.1e-7), Q6_K 2.0e-7 (2.1e-7).
 #pragma once
 
