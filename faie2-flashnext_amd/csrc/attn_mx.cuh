@@ -10,7 +10,7 @@
 // VALU for the split of K and V (11 instructions for two values), so the two are interleaved by hand: step s of the
 // walk issues 12 products on the operand split during step s - 1, and between them the 12 pieces of the split of step
 // s + 1's operand.  A step is 32 dims of a 16-key block's scores, or one 16-dim tile of P.V over 32 keys.  By the
-// counters of an 8-token step over 16 x 32K the matrix cores are busy 41 % of the time, the vector units 52 %, both at
+// counters of an 8-token step over 16 x 32K the matrix cores are busy 41 % of the time, the vector units 53 %, both at
 // once 17 %.
 // Contraction slots (free to permute as long as both operands agree), lane l, 8 a lane: of the scores, chunks 4 (2u)
 // + l/16 and 4 (2u + 1) + l/16 of the row (the cache's 16-byte chunks); of P.V, keys 4(l/16) + 0..3 of the first and
